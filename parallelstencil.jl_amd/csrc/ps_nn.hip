@@ -515,8 +515,15 @@ extern "C" int ps_nn_alloc(int64_t bytes, void** out) {
   void* p = nullptr;
   hipError_t e = hipMalloc(&p, (size_t)std::max<int64_t>(bytes, 256));
   if (e != hipSuccess) return ps_internal_fail(e == hipErrorOutOfMemory ? PS_EOOM : PS_EHIP, std::string("hipMalloc: ") + hipGetErrorString(e));
-  e = hipMemset(p, 0, (size_t)std::max<int64_t>(bytes, 256));
-  if (e != hipSuccess) return ps_internal_fail(PS_EHIP, std::string("hipMemset: ") + hipGetErrorString(e));
+  // cleared on the library's stream and waited for: a clear on the null stream is not ordered with the
+  // library's (non-blocking) streams and could land on what they write next
+  hipStream_t st = ps_internal_stream(nullptr);
+  e = hipMemsetAsync(p, 0, (size_t)std::max<int64_t>(bytes, 256), st);
+  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  if (e != hipSuccess) {
+    (void)hipFree(p);
+    return ps_internal_fail(PS_EHIP, std::string("ps_nn_alloc: ") + hipGetErrorString(e));
+  }
   *out = p;
   return 0;
 }
