@@ -22,6 +22,7 @@ namespace {
 typedef unsigned short bf16_t;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(8 * sizeof(short)))) short s16x8;
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short s16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 __device__ __forceinline__ float bf2f(bf16_t b) { return __uint_as_float((unsigned)b << 16); }
@@ -173,6 +174,182 @@ __global__ void __launch_bounds__(256) nn_gemm_k(int M, int N, int K, const bf16
           ((float*)C)[m * ldc + n] = v;
         }
       }
+}
+
+// ---- 3x3 convolution: the implicit im2col product with the input patch in LDS -------------------
+//
+// A workgroup owns a tile of TX columns x rows of one image's output pixels (16*MT*WM pixels) and
+// NB = 16*NT*WN output channels. The input patch of that tile (one pixel of halo, every channel) is
+// read from memory once into LDS, where all nine taps read it: the gather of nn_gemm_k reads it nine
+// times through L2. Only the weights are then staged, KS rows of them per barrier, double buffered.
+// The products take the pixels as the columns and the output channels as the rows of the MFMA, so
+// that a lane ends up with 4 consecutive channels of one pixel: one 8-byte store. The weights' operand
+// (8 consecutive k of one channel per lane) comes out of their [k][n] rows by the transposing LDS
+// read. k runs over tap*C + c in groups of 32 in ascending order, as in nn_gemm_k, so the sums are
+// bit for bit those of the stored column matrix.
+// Pixel stride in LDS: an odd number of 16-byte units, so that 16 lanes reading 16 bytes of 16
+// neighbouring pixels touch distinct banks.
+// With C below 8 (VEC false) the k of one 16-byte piece cross taps: the lane collects its 8 values
+// one by one from the patch.
+constexpr int KS = 64;
+
+__device__ __forceinline__ unsigned fdiv(unsigned e, unsigned d, unsigned magic) { return d == 1u ? e : __umulhi(e, magic); }
+
+__device__ __forceinline__ s16x4 lds_tr(const bf16_t* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+}
+__device__ __forceinline__ s16x8 cat8(s16x4 a, s16x4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+__device__ __forceinline__ f32x4 mfma(s16x8 a, s16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+template <int EPI, int MT, int NT, int WM, int WN, bool VEC>
+__global__ void __launch_bounds__(256) nn_conv3_k(const bf16_t* __restrict__ x, int H, int W, int C, const bf16_t* __restrict__ B, long long sbk,
+                                                  long long sbn, int N, bf16_t* __restrict__ Y, long long ldc, const float* __restrict__ bias,
+                                                  int lgTX, int tilesx, int tilesy, unsigned cmagic, unsigned pmagic) {
+  static_assert(WM * WN == 4, "four waves");
+  constexpr int NB = 16 * NT * WN, LDB = NB + 8, PB = KS * NB / 8 / 256;  // 16-byte pieces of a weight stage per thread
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
+  bf16_t* const Bs = lds;
+  bf16_t* const xs = lds + 2 * KS * LDB;
+  const int K = 9 * C, TX = 1 << lgTX, PW = TX + 2, rows = (16 * MT * WM) >> lgTX;
+  const int ps = VEC ? ((C >> 3) | 1) * 8 : C;  // LDS elements per patch pixel
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, li = lane & 15;
+  const int wm = WN == 1 ? w : w / WN, wn = WN == 1 ? 0 : w % WN;
+  int t = blockIdx.x;
+  const int tx0 = (t % tilesx) << lgTX;
+  t /= tilesx;
+  const int ty0 = (t % tilesy) * rows, img = t / tilesy;
+  const int n0 = blockIdx.y * NB;
+
+  const bool b_vec = sbn == 1 && sbk % 8 == 0 && ((uintptr_t)B & 15) == 0;
+  s16x8 pb[PB];
+  auto fetch_b = [&](int k0) {
+#pragma unroll
+    for (int j = 0; j < PB; ++j) {
+      const int q = tid + 256 * j, k = k0 + q / (NB / 8), n = n0 + (q % (NB / 8)) * 8;
+      if (b_vec && k < K && n + 7 < N) {
+        pb[j] = *(const s16x8*)(B + (long long)k * sbk + n);
+      } else {
+        for (int e = 0; e < 8; ++e) pb[j][e] = (k < K && n + e < N) ? (short)B[(long long)k * sbk + (long long)(n + e) * sbn] : (short)0;
+      }
+    }
+  };
+  auto store_b = [&](int buf) {
+#pragma unroll
+    for (int j = 0; j < PB; ++j) {
+      const int q = tid + 256 * j;
+      *(s16x8*)&Bs[(buf * KS + q / (NB / 8)) * LDB + (q % (NB / 8)) * 8] = pb[j];
+    }
+  };
+  fetch_b(0);
+  {  // the patch: rows + 2 by TX + 2 pixels, zero outside the image
+    const unsigned cp = VEC ? (unsigned)C >> 3 : (unsigned)C, total = (unsigned)((rows + 2) * PW) * cp;
+    const long long base = (long long)img * H * W;
+    for (unsigned e0 = tid; e0 < total; e0 += 4 * 256) {
+      s16x8 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const unsigned e = e0 + 256 * u;
+        v[u] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        if (e < total) {
+          const unsigned p = fdiv(e, cp, cmagic), c = e - p * cp, py = fdiv(p, (unsigned)PW, pmagic);
+          const int yy = ty0 + (int)py - 1, xx = tx0 + (int)(p - py * PW) - 1;
+          if (yy >= 0 && yy < H && xx >= 0 && xx < W) {
+            const bf16_t* src = x + (base + (long long)yy * W + xx) * C;
+            if (VEC) v[u] = *(const s16x8*)(src + c * 8);
+            else v[u][0] = (short)src[c];
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const unsigned e = e0 + 256 * u;
+        if (e < total) {
+          const unsigned p = fdiv(e, cp, cmagic), c = e - p * cp;
+          if (VEC) *(s16x8*)&xs[p * ps + c * 8] = v[u];
+          else xs[e] = (bf16_t)v[u][0];
+        }
+      }
+    }
+  }
+  store_b(0);
+  int px[MT];  // the patch element where the window of this lane's pixel of M tile i starts
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int q = (wm * MT + i) * 16 + li;
+    px[i] = ((q >> lgTX) * PW + (q & (TX - 1))) * ps;
+  }
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+  for (int s = 0; s * KS < K; ++s) {
+    const bool more = (s + 1) * KS < K;
+    if (more) fetch_b((s + 1) * KS);
+#pragma unroll
+    for (int kk = 0; kk < KS; kk += 32) {
+      const int k0 = s * KS + kk;
+      if (k0 < K) {
+        s16x8 a[NT], b[MT];
+        const bf16_t* bp = &Bs[((s & 1) * KS + kk + 8 * g + (li >> 2)) * LDB + wn * NT * 16 + 4 * (li & 3)];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) a[j] = cat8(lds_tr(bp + 16 * j), lds_tr(bp + 16 * j + 4 * LDB));
+        if (VEC) {
+          const unsigned k = k0 + 8 * g, tap = fdiv(k >> 3, (unsigned)C >> 3, cmagic), ky = (tap * 11u) >> 5;
+          const int off = (int)((ky * PW + (tap - 3 * ky)) * ps + (k - tap * C));
+          const bool in = k < (unsigned)K;
+#pragma unroll
+          for (int i = 0; i < MT; ++i) {
+            b[i] = *(const s16x8*)&xs[in ? px[i] + off : px[i]];
+            if (!in) b[i] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const unsigned k = k0 + 8 * g + e, tap = fdiv(k, (unsigned)C, cmagic), ky = (tap * 11u) >> 5;
+            const int off = (int)((ky * PW + (tap - 3 * ky)) * ps + (k - tap * C));
+            const bool in = k < (unsigned)K;
+#pragma unroll
+            for (int i = 0; i < MT; ++i) b[i][e] = in ? (short)xs[px[i] + off] : (short)0;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int j = 0; j < NT; ++j) acc[i][j] = mfma(a[j], b[i], acc[i][j]);
+      }
+    }
+    if (more) store_b((s + 1) & 1);
+    __syncthreads();
+  }
+  const bool c_vec = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)Y & 7) == 0;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int q = (wm * MT + i) * 16 + li, yy = ty0 + (q >> lgTX), xx = tx0 + (q & (TX - 1));
+    if (yy >= H || xx >= W) continue;
+    bf16_t* const yp = Y + (((long long)img * H + yy) * W + xx) * ldc;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int n = n0 + (wn * NT + j) * 16 + 4 * g;
+      s16x4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v = acc[i][j][r];
+        if (EPI != PS_NN_EPI_BF16) v += n + r < N ? bias[n + r] : 0.f;
+        if (EPI == PS_NN_EPI_BF16_BIAS_RELU) v = v > 0.f ? v : 0.f;
+        o[r] = (short)f2bf(v);
+      }
+      if (c_vec) {
+        if (n < N) *(s16x4*)(yp + n) = o;
+      } else {
+        for (int r = 0; r < 4; ++r)
+          if (n + r < N) yp[n + r] = (bf16_t)o[r];
+      }
+    }
+  }
 }
 
 unsigned grid_for(long long n) { return (unsigned)std::min<long long>((n + 255) / 256, 1 << 20); }
@@ -408,6 +585,59 @@ int gemm_launch(int M, int N, int K, const void* A, int64_t sam, int64_t sak, co
   return launched("ps_nn_gemm");
 }
 
+// The 3x3 convolution with the patch in LDS (nn_conv3_k), or 1 where the general product serves:
+// FP32 results and split K, 8 channels and more that are not whole aligned 16-byte pieces, and
+// channel counts whose patch does not fit the LDS.
+int conv3_launch(int M, int N, const bf16_t* x, int H, int W, int C, const bf16_t* B, long long sbk, long long sbn, void* Cm, long long ldc,
+                 const float* bias, int epi, int splitk, hipStream_t st) {
+  const bool vec = C % 8 == 0;
+  if (splitk != 1 || (epi != PS_NN_EPI_BF16 && epi != PS_NN_EPI_BF16_BIAS_RELU && epi != PS_NN_EPI_BF16_BIAS)) return 1;
+  if (!(vec && ((uintptr_t)x & 15) == 0) && C >= 8) return 1;
+  const long long imgs = M / ((long long)H * W);
+  auto up = [](long long a, long long b) { return (a + b - 1) / b; };
+  // pixel tiles of 16 x 16 (64 pixels: 16 x 4), or 8 columns wide where that pads the image less
+  auto shape = [&](int pix, int& lg) -> long long {
+    const long long w16 = up(W, 16) * up(H, pix / 16), w8 = up(W, 8) * up(H, pix / 8);
+    lg = w8 < w16 ? 3 : 4;
+    return std::min(w16, w8) * imgs;
+  };
+  const int nb = N <= 32 ? 32 : 64;
+  int lg = 4;
+  int pix = 256;
+  // 256 pixels a workgroup while that leaves two workgroups for every CU, 64 pixels below
+  long long tiles = shape(256, lg);
+  auto lds = [&](int px, int lgx) {
+    const long long ps = vec ? ((C >> 3) | 1) * 8 : C;
+    return 2LL * (2 * KS * (nb + 8) + ((px >> lgx) + 2) * ((1 << lgx) + 2) * ps);
+  };
+  if (tiles * up(N, nb) < 512 || lds(256, lg) > 81920) {
+    pix = 64;
+    tiles = shape(64, lg);
+  }
+  if (lds(pix, lg) > 160 * 1024 || tiles > 0x7fffffffLL || up(N, nb) > 65535) return 1;
+  const int tx = 1 << lg, rows = pix / tx, tilesx = (int)up(W, tx), tilesy = (int)up(H, rows);
+  const unsigned d = vec ? (unsigned)C >> 3 : (unsigned)C;
+  const unsigned cmagic = d == 1 ? 0u : (unsigned)((0x100000000ULL + d - 1) / d), pmagic = (unsigned)((0x100000000ULL + tx + 1) / (tx + 2));
+  const dim3 grid((unsigned)tiles, (unsigned)up(N, nb));
+  const size_t sh = (size_t)lds(pix, lg);
+#define NN_CONV3(E, MT, NT, WM, WN)                                                                                                              if (vec) hipLaunchKernelGGL((nn_conv3_k<E, MT, NT, WM, WN, true>), grid, dim3(256), sh, st, x, H, W, C, B, sbk, sbn, N, (bf16_t*)Cm, ldc, bias, lg,                               tilesx, tilesy, cmagic, pmagic);                                                                                   else hipLaunchKernelGGL((nn_conv3_k<E, MT, NT, WM, WN, false>), grid, dim3(256), sh, st, x, H, W, C, B, sbk, sbn, N, (bf16_t*)Cm, ldc, bias, lg,                              tilesx, tilesy, cmagic, pmagic);
+#define NN_CONV3_CASE(E)                               \
+  case E:                                              \
+    if (pix == 256 && nb == 64) { NN_CONV3(E, 4, 4, 4, 1) } \
+    else if (pix == 256) { NN_CONV3(E, 4, 2, 4, 1) }   \
+    else if (nb == 64) { NN_CONV3(E, 2, 2, 2, 2) }     \
+    else { NN_CONV3(E, 1, 2, 4, 1) }                   \
+    break;
+  switch (epi) {
+    NN_CONV3_CASE(PS_NN_EPI_BF16)
+    NN_CONV3_CASE(PS_NN_EPI_BF16_BIAS_RELU)
+    NN_CONV3_CASE(PS_NN_EPI_BF16_BIAS)
+  }
+#undef NN_CONV3_CASE
+#undef NN_CONV3
+  return launched("ps_nn_gemm_im2col");
+}
+
 }  // namespace
 
 extern "C" int ps_nn_gemm(int M, int N, int K, const void* A, int64_t sam, int64_t sak, const void* B, int64_t sbk, int64_t sbn, void* C,
@@ -423,6 +653,10 @@ extern "C" int ps_nn_gemm_im2col(int transpose, int M, int N, int K, const void*
   const long long npix = transpose ? (long long)K : (long long)M, ncol = transpose ? (long long)M : (long long)K;
   if (ncol != 9LL * Cin || npix % ((long long)H * W) != 0)
     return ps_internal_fail(PS_EARGUMENT, "ps_nn_gemm_im2col: the im2col operand is (B*H*W) x (9*C): sizes do not match");
+  if (!transpose && M > 0 && N > 0 && (epi == PS_NN_EPI_BF16 || bias)) {
+    const int r = conv3_launch(M, N, (const bf16_t*)x, H, W, Cin, (const bf16_t*)B, sbk, sbn, C, ldc, bias, epi, splitk, st);
+    if (r <= 0) return r;
+  }
   return transpose ? gemm_launch<2>(M, N, K, x, 0, 0, B, sbk, sbn, C, ldc, bias, epi, splitk, st, H, W, Cin)
                    : gemm_launch<1>(M, N, K, x, 0, 0, B, sbk, sbn, C, ldc, bias, epi, splitk, st, H, W, Cin);
 }
@@ -512,12 +746,16 @@ extern "C" int ps_nn_add_bf16(void* y, const void* x, int64_t n, void* stream) {
 extern "C" int ps_nn_alloc(int64_t bytes, void** out) {
   if (int r = ps_internal_require_init()) return r;
   if (bytes < 0) return ps_internal_fail(PS_EARGUMENT, "ps_nn_alloc: negative size");
+  hipStream_t st = ps_internal_stream(nullptr);
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  hipError_t e = hipStreamIsCapturing(st, &cs);
+  if (e == hipSuccess && cs != hipStreamCaptureStatusNone)
+    return ps_internal_fail(PS_EARGUMENT, "ps_nn_alloc: cannot allocate while a graph is being captured on the library stream");
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, (size_t)std::max<int64_t>(bytes, 256));
+  e = hipMalloc(&p, (size_t)std::max<int64_t>(bytes, 256));
   if (e != hipSuccess) return ps_internal_fail(e == hipErrorOutOfMemory ? PS_EOOM : PS_EHIP, std::string("hipMalloc: ") + hipGetErrorString(e));
   // cleared on the library's stream and waited for: a clear on the null stream is not ordered with the
   // library's (non-blocking) streams and could land on what they write next
-  hipStream_t st = ps_internal_stream(nullptr);
   e = hipMemsetAsync(p, 0, (size_t)std::max<int64_t>(bytes, 256), st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e != hipSuccess) {
