@@ -192,6 +192,7 @@ __global__ void __launch_bounds__(256) nn_gemm_k(int M, int N, int K, const bf16
 // With C below 8 (VEC false) the k of one 16-byte piece cross taps: the lane collects its 8 values
 // one by one from the patch.
 constexpr int KS = 64;
+constexpr int KD = 2;  // weight stages in flight ahead of the one in LDS (even: stage s goes through LDS buffer s & 1)
 
 __device__ __forceinline__ unsigned fdiv(unsigned e, unsigned d, unsigned magic) { return d == 1u ? e : __umulhi(e, magic); }
 
@@ -202,13 +203,24 @@ __device__ __forceinline__ s16x8 cat8(s16x4 a, s16x4 b) { return __builtin_shuff
 __device__ __forceinline__ f32x4 mfma(s16x8 a, s16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
+// f2bf of 4 values, by the rounding instruction (which keeps a NaN's payload: NaNs become 0x7fc00000 first)
+__device__ __forceinline__ s16x4 f2bf4(f32x4 v) {
+  typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = v[r] == v[r] ? v[r] : __uint_as_float(0x7fc00000u);
+  return __builtin_bit_cast(s16x4, __builtin_convertvector(v, bf16x4));
+}
 
-template <int EPI, int MT, int NT, int WM, int WN, bool VEC>
-__global__ void __launch_bounds__(256) nn_conv3_k(const bf16_t* __restrict__ x, int H, int W, int C, const bf16_t* __restrict__ B, long long sbk,
-                                                  long long sbn, int N, bf16_t* __restrict__ Y, long long ldc, const float* __restrict__ bias,
-                                                  int lgTX, int tilesx, int tilesy, unsigned cmagic, unsigned pmagic) {
-  static_assert(WM * WN == 4, "four waves");
-  constexpr int NB = 16 * NT * WN, LDB = NB + 8, PB = KS * NB / 8 / 256;  // 16-byte pieces of a weight stage per thread
+// MODE: 0 C below 8, 1 C a multiple of 8, 2 C a multiple of 32 (a group of 32 k stays in one tap, whose
+// place in the patch is then the same for all lanes)
+template <int EPI, int MT, int NT, int WM, int WN, int MODE>
+__global__ void __launch_bounds__(64 * WM * WN) nn_conv3_k(const bf16_t* __restrict__ x, int H, int W, int C, const bf16_t* __restrict__ B,
+                                                           long long sbk, long long sbn, int N, bf16_t* __restrict__ Y, int ldc,
+                                                           const float* __restrict__ bias, int lgTX, int tilesx, int tilesy, unsigned cmagic,
+                                                           unsigned pmagic) {
+  constexpr bool VEC = MODE != 0;
+  constexpr int NTH = 64 * WM * WN, NB = 16 * NT * WN, LDB = NB + 8;
+  constexpr int PIECES = KS * NB / 8, PB = (PIECES + NTH - 1) / NTH;  // 16-byte pieces of a weight stage, and per thread
   extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
   bf16_t* const Bs = lds;
   bf16_t* const xs = lds + 2 * KS * LDB;
@@ -222,126 +234,173 @@ __global__ void __launch_bounds__(256) nn_conv3_k(const bf16_t* __restrict__ x, 
   const int ty0 = (t % tilesy) * rows, img = t / tilesy;
   const int n0 = blockIdx.y * NB;
 
-  const bool b_vec = sbn == 1 && sbk % 8 == 0 && ((uintptr_t)B & 15) == 0;
-  s16x8 pb[PB];
-  auto fetch_b = [&](int k0) {
+  // weights: piece j of this thread holds columns bn.. of row bk + s*KS in stage s
+  s16x8 pb[KD][PB];
+  const bf16_t* bptr[PB];
+  bool bfull[PB];
+  int bk[PB], bn[PB], bl[PB];
+#pragma unroll
+  for (int j = 0; j < PB; ++j) {
+    const int q = tid + NTH * j;
+    bk[j] = PIECES % NTH == 0 || q < PIECES ? q / (NB / 8) : 1 << 30;
+    bn[j] = n0 + (q % (NB / 8)) * 8;
+    bl[j] = (q / (NB / 8)) * LDB + (q % (NB / 8)) * 8;
+    bptr[j] = B + (long long)(q / (NB / 8)) * sbk + (long long)bn[j] * sbn;
+    bfull[j] = sbn == 1 && sbk % 8 == 0 && ((uintptr_t)B & 15) == 0 && bn[j] + 7 < N;
+  }
+  auto fetch_b = [&](s16x8 (&v)[PB], int k0) {
 #pragma unroll
     for (int j = 0; j < PB; ++j) {
-      const int q = tid + 256 * j, k = k0 + q / (NB / 8), n = n0 + (q % (NB / 8)) * 8;
-      if (b_vec && k < K && n + 7 < N) {
-        pb[j] = *(const s16x8*)(B + (long long)k * sbk + n);
-      } else {
-        for (int e = 0; e < 8; ++e) pb[j][e] = (k < K && n + e < N) ? (short)B[(long long)k * sbk + (long long)(n + e) * sbn] : (short)0;
+      v[j] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (k0 + bk[j] < K) {
+        const bf16_t* const p = bptr[j] + (long long)k0 * sbk;
+        if (bfull[j]) {
+          v[j] = *(const s16x8*)p;
+        } else {
+          for (int e = 0; e < 8; ++e)
+            if (bn[j] + e < N) v[j][e] = (short)p[e * sbn];
+        }
       }
     }
   };
-  auto store_b = [&](int buf) {
+  auto store_b = [&](const s16x8 (&v)[PB], int buf) {
 #pragma unroll
-    for (int j = 0; j < PB; ++j) {
-      const int q = tid + 256 * j;
-      *(s16x8*)&Bs[(buf * KS + q / (NB / 8)) * LDB + (q % (NB / 8)) * 8] = pb[j];
-    }
+    for (int j = 0; j < PB; ++j)
+      if (PIECES % NTH == 0 || tid + NTH * j < PIECES) *(s16x8*)&Bs[buf * KS * LDB + bl[j]] = v[j];
   };
-  fetch_b(0);
-  {  // the patch: rows + 2 by TX + 2 pixels, zero outside the image
+#pragma unroll
+  for (int d = 0; d < KD; ++d) fetch_b(pb[d], d * KS);
+  {  // the patch, PU pieces per thread in flight: rows + 2 by TX + 2 pixels, zero outside the image
+    constexpr int PU = 4;
     const unsigned cp = VEC ? (unsigned)C >> 3 : (unsigned)C, total = (unsigned)((rows + 2) * PW) * cp;
-    const long long base = (long long)img * H * W;
-    for (unsigned e0 = tid; e0 < total; e0 += 4 * 256) {
-      s16x8 v[4];
+    const char* const xi = (const char*)(x + (long long)img * H * W * C);  // the launch checks that an image is below 4 GB
+    for (unsigned e0 = tid; e0 < total; e0 += PU * NTH) {
+      s16x8 v[PU];
+      unsigned at[PU];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const unsigned e = e0 + 256 * u;
+      for (int u = 0; u < PU; ++u) {
+        const unsigned e = e0 + NTH * u, p = fdiv(e, cp, cmagic), c = e - p * cp, py = fdiv(p, (unsigned)PW, pmagic);
+        const int yy = ty0 + (int)py - 1, xx = tx0 + (int)(p - py * PW) - 1;
+        at[u] = p * ps + (VEC ? c * 8 : c);
         v[u] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        if (e < total) {
-          const unsigned p = fdiv(e, cp, cmagic), c = e - p * cp, py = fdiv(p, (unsigned)PW, pmagic);
-          const int yy = ty0 + (int)py - 1, xx = tx0 + (int)(p - py * PW) - 1;
-          if (yy >= 0 && yy < H && xx >= 0 && xx < W) {
-            const bf16_t* src = x + (base + (long long)yy * W + xx) * C;
-            if (VEC) v[u] = *(const s16x8*)(src + c * 8);
-            else v[u][0] = (short)src[c];
-          }
+        if (e < total && (unsigned)yy < (unsigned)H && (unsigned)xx < (unsigned)W) {
+          const char* const src = xi + (size_t)(((unsigned)yy * (unsigned)W + (unsigned)xx) * (unsigned)(2 * C) + c * (VEC ? 16u : 2u));
+          if (VEC) v[u] = *(const s16x8*)src;
+          else v[u][0] = *(const short*)src;
         }
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const unsigned e = e0 + 256 * u;
-        if (e < total) {
-          const unsigned p = fdiv(e, cp, cmagic), c = e - p * cp;
-          if (VEC) *(s16x8*)&xs[p * ps + c * 8] = v[u];
-          else xs[e] = (bf16_t)v[u][0];
+      for (int u = 0; u < PU; ++u)
+        if (e0 + NTH * u < total) {
+          if (VEC) *(s16x8*)&xs[at[u]] = v[u];
+          else xs[at[u]] = (bf16_t)v[u][0];
         }
-      }
     }
   }
-  store_b(0);
+  store_b(pb[0], 0);
+  fetch_b(pb[0], KD * KS);
   int px[MT];  // the patch element where the window of this lane's pixel of M tile i starts
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int q = (wm * MT + i) * 16 + li;
-    px[i] = ((q >> lgTX) * PW + (q & (TX - 1))) * ps;
+    px[i] = ((q >> lgTX) * PW + (q & (TX - 1))) * ps + (MODE == 2 ? 8 * g : 0);
   }
   f32x4 acc[MT][NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 bv[NT];
+  if (EPI != PS_NN_EPI_BF16) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int n = n0 + (wn * NT + j) * 16 + 4 * g + r;
+        bv[j][r] = n < N ? bias[n] : 0.f;
+      }
+  }
+  const bf16_t* const bp0 = &Bs[(8 * g + (li >> 2)) * LDB + wn * NT * 16 + 4 * (li & 3)];
+  int tap = 0, c0 = 0;  // MODE 2: tap and first channel of the group
   __syncthreads();
-  for (int s = 0; s * KS < K; ++s) {
-    const bool more = (s + 1) * KS < K;
-    if (more) fetch_b((s + 1) * KS);
+  for (int s0 = 0; s0 * KS < K; s0 += KD) {
 #pragma unroll
-    for (int kk = 0; kk < KS; kk += 32) {
-      const int k0 = s * KS + kk;
-      if (k0 < K) {
-        s16x8 a[NT], b[MT];
-        const bf16_t* bp = &Bs[((s & 1) * KS + kk + 8 * g + (li >> 2)) * LDB + wn * NT * 16 + 4 * (li & 3)];
+    for (int d = 0; d < KD; ++d) {
+      const int s = s0 + d;
+      if (s * KS >= K) break;
 #pragma unroll
-        for (int j = 0; j < NT; ++j) a[j] = cat8(lds_tr(bp + 16 * j), lds_tr(bp + 16 * j + 4 * LDB));
-        if (VEC) {
-          const unsigned k = k0 + 8 * g, tap = fdiv(k >> 3, (unsigned)C >> 3, cmagic), ky = (tap * 11u) >> 5;
-          const int off = (int)((ky * PW + (tap - 3 * ky)) * ps + (k - tap * C));
-          const bool in = k < (unsigned)K;
+      for (int kk = 0; kk < KS; kk += 32) {
+        const int k0 = s * KS + kk;
+        if (k0 < K) {
+          s16x8 a[NT], b[MT];
+          const bf16_t* const bp = bp0 + ((d & 1) * KS + kk) * LDB;
 #pragma unroll
-          for (int i = 0; i < MT; ++i) {
-            b[i] = *(const s16x8*)&xs[in ? px[i] + off : px[i]];
-            if (!in) b[i] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+          for (int j = 0; j < NT; ++j) a[j] = cat8(lds_tr(bp + 16 * j), lds_tr(bp + 16 * j + 4 * LDB));
+          if (MODE == 2) {
+            const int ky = (tap * 11) >> 5, off = (ky * PW + (tap - 3 * ky)) * ps + c0;
+#pragma unroll
+            for (int i = 0; i < MT; ++i) b[i] = *(const s16x8*)&xs[px[i] + off];
+            c0 += 32;
+            if (c0 == C) {
+              c0 = 0;
+              ++tap;
+            }
+          } else if (MODE == 1) {
+            const unsigned k = k0 + 8 * g, tp = fdiv(k >> 3, (unsigned)C >> 3, cmagic), ky = (tp * 11u) >> 5;
+            const int off = (int)((ky * PW + (tp - 3 * ky)) * ps + (k - tp * C));
+            if (k0 + 32 <= K) {
+#pragma unroll
+              for (int i = 0; i < MT; ++i) b[i] = *(const s16x8*)&xs[px[i] + off];
+            } else {  // the last group of a K that is no multiple of 32: zeros behind it
+#pragma unroll
+              for (int i = 0; i < MT; ++i) {
+                b[i] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+                if (k < (unsigned)K) b[i] = *(const s16x8*)&xs[px[i] + off];
+              }
+            }
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const unsigned k = k0 + 8 * g + e, tp = fdiv(k, (unsigned)C, cmagic), ky = (tp * 11u) >> 5;
+              const int off = (int)((ky * PW + (tp - 3 * ky)) * ps + (k - tp * C));
+              const bool in = k < (unsigned)K;
+#pragma unroll
+              for (int i = 0; i < MT; ++i) b[i][e] = in ? (short)xs[px[i] + off] : (short)0;
+            }
           }
-        } else {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const unsigned k = k0 + 8 * g + e, tap = fdiv(k, (unsigned)C, cmagic), ky = (tap * 11u) >> 5;
-            const int off = (int)((ky * PW + (tap - 3 * ky)) * ps + (k - tap * C));
-            const bool in = k < (unsigned)K;
+          for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int i = 0; i < MT; ++i) b[i][e] = in ? (short)xs[px[i] + off] : (short)0;
-          }
+            for (int j = 0; j < NT; ++j) acc[i][j] = mfma(a[j], b[i], acc[i][j]);
         }
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int j = 0; j < NT; ++j) acc[i][j] = mfma(a[j], b[i], acc[i][j]);
+      }
+      if ((s + 1) * KS < K) {
+        // stage s + 1 goes to the buffer that stage s - 1 was read from before the last barrier
+        store_b(pb[(d + 1) % KD], (d + 1) & 1);
+        fetch_b(pb[(d + 1) % KD], (s + 1 + KD) * KS);
+        __syncthreads();
       }
     }
-    if (more) store_b((s + 1) & 1);
-    __syncthreads();
   }
   const bool c_vec = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)Y & 7) == 0;
+  bf16_t* const yi = Y + (long long)img * H * W * ldc;
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int q = (wm * MT + i) * 16 + li, yy = ty0 + (q >> lgTX), xx = tx0 + (q & (TX - 1));
     if (yy >= H || xx >= W) continue;
-    bf16_t* const yp = Y + (((long long)img * H + yy) * W + xx) * ldc;
+    bf16_t* const yp = yi + (size_t)(((unsigned)yy * (unsigned)W + (unsigned)xx) * (unsigned)ldc);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const int n = n0 + (wn * NT + j) * 16 + 4 * g;
-      s16x4 o;
+      f32x4 v = acc[i][j];
+      if (EPI != PS_NN_EPI_BF16) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float v = acc[i][j][r];
-        if (EPI != PS_NN_EPI_BF16) v += n + r < N ? bias[n + r] : 0.f;
-        if (EPI == PS_NN_EPI_BF16_BIAS_RELU) v = v > 0.f ? v : 0.f;
-        o[r] = (short)f2bf(v);
+        for (int r = 0; r < 4; ++r) {
+          v[r] += bv[j][r];
+          if (EPI == PS_NN_EPI_BF16_BIAS_RELU) v[r] = v[r] > 0.f ? v[r] : 0.f;
+        }
       }
+      const s16x4 o = f2bf4(v);
       if (c_vec) {
         if (n < N) *(s16x4*)(yp + n) = o;
       } else {
@@ -593,40 +652,63 @@ int conv3_launch(int M, int N, const bf16_t* x, int H, int W, int C, const bf16_
   const bool vec = C % 8 == 0;
   if (splitk != 1 || (epi != PS_NN_EPI_BF16 && epi != PS_NN_EPI_BF16_BIAS_RELU && epi != PS_NN_EPI_BF16_BIAS)) return 1;
   if (!(vec && ((uintptr_t)x & 15) == 0) && C >= 8) return 1;
+  // offsets inside one image are 32-bit
+  if ((long long)H * W > 0x7fffffffLL / std::max<long long>(C, std::max<long long>(ldc, N)) || ldc < 0) return 1;
+  const int mode = !vec ? 0 : C % 32 == 0 ? 2 : 1;
   const long long imgs = M / ((long long)H * W);
   auto up = [](long long a, long long b) { return (a + b - 1) / b; };
-  // pixel tiles of 16 x 16 (64 pixels: 16 x 4), or 8 columns wide where that pads the image less
+  // pixel tiles 16 columns wide, or 8 where that pads the image less
   auto shape = [&](int pix, int& lg) -> long long {
     const long long w16 = up(W, 16) * up(H, pix / 16), w8 = up(W, 8) * up(H, pix / 8);
     lg = w8 < w16 ? 3 : 4;
     return std::min(w16, w8) * imgs;
   };
-  const int nb = N <= 32 ? 32 : 64;
-  int lg = 4;
-  int pix = 256;
-  // 256 pixels a workgroup while that leaves two workgroups for every CU, 64 pixels below
-  long long tiles = shape(256, lg);
-  auto lds = [&](int px, int lgx) {
+  // Tile (pixels x channels, 8 wavefronts each). While the patch leaves room for two workgroups on a
+  // CU, 256 x 32: the most workgroups in flight, so that one's loads run under another's products
+  // (32 -> 32 at 512^2: 18.6 us; 256 x 64 with the padded channels 25.2, four wavefronts 20.4). Where
+  // it does not (C = 128 and above), the patch is better read by fewer workgroups: 256 x 64, then
+  // 128 x 64 (192 -> 64 at 256^2: 28.6 us against 41.1 with 256 x 32; 384 -> 128 at 128^2: 34.9
+  // against 52.9 with 128 x 32). Tiles that leave CUs without a workgroup give way to smaller ones
+  // (256 -> 256 at 64^2: 128 x 32 20.0 us, 128 x 64 24.8). What then bounded the small-C layers was
+  // vector instructions around the products (index quotients, masks, rounding): with the patch place
+  // of a group of 32 k in scalar registers (MODE 2) and the rounding instruction, 32 -> 32 at 512^2
+  // runs 13.8 us, 192 -> 64 26.5, 384 -> 128 31.8.
+  struct Tile { int pix, nb; };
+  static const Tile tiles[4] = {{256, 64}, {128, 64}, {256, 32}, {128, 32}};
+  int lg = 4, pick = -1;
+  long long ntile = 0, lds = 0;
+  auto fits = [&](int v) {
     const long long ps = vec ? ((C >> 3) | 1) * 8 : C;
-    return 2LL * (2 * KS * (nb + 8) + ((px >> lgx) + 2) * ((1 << lgx) + 2) * ps);
+    ntile = shape(tiles[v].pix, lg);
+    lds = 2LL * (2 * KS * (tiles[v].nb + 8) + ((tiles[v].pix >> lg) + 2) * ((1 << lg) + 2) * ps);
+    return lds <= 160 * 1024;
   };
-  if (tiles * up(N, nb) < 512 || lds(256, lg) > 81920) {
-    pix = 64;
-    tiles = shape(64, lg);
-  }
-  if (lds(pix, lg) > 160 * 1024 || tiles > 0x7fffffffLL || up(N, nb) > 65535) return 1;
-  const int tx = 1 << lg, rows = pix / tx, tilesx = (int)up(W, tx), tilesy = (int)up(H, rows);
+  const bool two = fits(2) && lds <= 80 * 1024;
+  for (int v = two ? 2 : 0; v < 4 && pick < 0; ++v)
+    if (fits(v) && (v == 3 || ntile * up(N, tiles[v].nb) >= 256)) pick = v;
+  if (pick < 0) return 1;
+  const int pix = tiles[pick].pix, nb = tiles[pick].nb;
+  if (ntile > 0x7fffffffLL || up(N, nb) > 65535) return 1;
+  const int tx = 1 << lg, tilesx = (int)up(W, tx), tilesy = (int)up(H, pix / tx);
   const unsigned d = vec ? (unsigned)C >> 3 : (unsigned)C;
   const unsigned cmagic = d == 1 ? 0u : (unsigned)((0x100000000ULL + d - 1) / d), pmagic = (unsigned)((0x100000000ULL + tx + 1) / (tx + 2));
-  const dim3 grid((unsigned)tiles, (unsigned)up(N, nb));
-  const size_t sh = (size_t)lds(pix, lg);
-#define NN_CONV3(E, MT, NT, WM, WN)                                                                                                              if (vec) hipLaunchKernelGGL((nn_conv3_k<E, MT, NT, WM, WN, true>), grid, dim3(256), sh, st, x, H, W, C, B, sbk, sbn, N, (bf16_t*)Cm, ldc, bias, lg,                               tilesx, tilesy, cmagic, pmagic);                                                                                   else hipLaunchKernelGGL((nn_conv3_k<E, MT, NT, WM, WN, false>), grid, dim3(256), sh, st, x, H, W, C, B, sbk, sbn, N, (bf16_t*)Cm, ldc, bias, lg,                              tilesx, tilesy, cmagic, pmagic);
-#define NN_CONV3_CASE(E)                               \
-  case E:                                              \
-    if (pix == 256 && nb == 64) { NN_CONV3(E, 4, 4, 4, 1) } \
-    else if (pix == 256) { NN_CONV3(E, 4, 2, 4, 1) }   \
-    else if (nb == 64) { NN_CONV3(E, 2, 2, 2, 2) }     \
-    else { NN_CONV3(E, 1, 2, 4, 1) }                   \
+  const dim3 grid((unsigned)ntile, (unsigned)up(N, nb));
+#define NN_CONV3(E, MT, NT, WM, WN, MODE)                                                                                                       \
+  hipLaunchKernelGGL((nn_conv3_k<E, MT, NT, WM, WN, MODE>), grid, dim3(512), (size_t)lds, st, x, H, W, C, B, sbk, sbn, N, (bf16_t*)Cm, (int)ldc, bias, \
+                     lg, tilesx, tilesy, cmagic, pmagic)
+#define NN_CONV3_TILE(E, MT, NT, WM, WN)              \
+  {                                                   \
+    if (mode == 2) NN_CONV3(E, MT, NT, WM, WN, 2);    \
+    else NN_CONV3(E, MT, NT, WM, WN, 1);              \
+  }
+#define NN_CONV3_CASE(E)                              \
+  case E:                                             \
+    if (pick == 2 && !vec) NN_CONV3(E, 2, 2, 8, 1, 0); \
+    else if (!vec) NN_CONV3(E, 1, 2, 8, 1, 0);        \
+    else if (pick == 0) NN_CONV3_TILE(E, 2, 4, 8, 1)  \
+    else if (pick == 1) NN_CONV3_TILE(E, 2, 2, 4, 2)  \
+    else if (pick == 2) NN_CONV3_TILE(E, 2, 2, 8, 1)  \
+    else NN_CONV3_TILE(E, 1, 2, 8, 1)                 \
     break;
   switch (epi) {
     NN_CONV3_CASE(PS_NN_EPI_BF16)
@@ -634,6 +716,7 @@ int conv3_launch(int M, int N, const bf16_t* x, int H, int W, int C, const bf16_
     NN_CONV3_CASE(PS_NN_EPI_BF16_BIAS)
   }
 #undef NN_CONV3_CASE
+#undef NN_CONV3_TILE
 #undef NN_CONV3
   return launched("ps_nn_gemm_im2col");
 }
