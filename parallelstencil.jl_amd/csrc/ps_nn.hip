@@ -449,95 +449,109 @@ __global__ void __launch_bounds__(256) nn_col2im_k(const bf16_t* __restrict__ dc
   }
 }
 
-__global__ void __launch_bounds__(256) nn_pool2_k(const bf16_t* __restrict__ x, int B, int H, int W, int C, bf16_t* __restrict__ y) {
-  const int Ho = H / 2, Wo = W / 2;
-  const long long n = (long long)B * Ho * Wo * C;
+// The data movement of the network between its products: V channels (8: 16 bytes, where the channel
+// counts and the pointers allow it) per thread. One element per thread was bound by its 64-bit
+// index quotients, not by memory: up2 of 1 x 256^2 x 64 took 57.9 us (0.72 TB/s), 8 channels a
+// thread 7.1 (5.9 TB/s).
+template <int V>
+struct Piece {
+  bf16_t v[V];
+};
+template <>
+struct __attribute__((aligned(16))) Piece<8> {
+  bf16_t v[8];
+};
+
+// Low-resolution piece e of (B, H, W, C) and the four pieces of its 2x2 pixels in (B, 2H, 2W, C):
+// OP 0 average pooling (four in, one out), 1 its adjoint, 2 nearest upsampling (one in, four out),
+// 3 its adjoint. blockIdx.y strides over the B*H rows, x over the pieces of a row.
+template <int OP, int V>
+__global__ void __launch_bounds__(256) nn_quad_k(const bf16_t* __restrict__ in, long long rows, int W, int C, bf16_t* __restrict__ out) {
+  const unsigned cp = (unsigned)C / V;  // pieces of a pixel
+  const long long rp = (long long)W * cp;  // and of a low-resolution row
+  const Piece<V>* const src = (const Piece<V>*)in;
+  Piece<V>* const dst = (Piece<V>*)out;
+  GS_LOOP(e, rp) {
+    const long long xx = rp <= 0xffffffffLL ? (long long)((unsigned)e / cp) : e / cp, c = e - xx * cp;
+    for (long long r = blockIdx.y; r < rows; r += gridDim.y) {
+      const long long lo = r * rp + e, hi = 4 * r * rp + 2 * xx * cp + c;  // rows 2r and 2r + 1 hold 2*rp pieces each
+      const long long h[4] = {hi, hi + cp, hi + 2 * rp, hi + 2 * rp + cp};
+      if (OP == 0 || OP == 3) {
+        const Piece<V> a = src[h[0]], b = src[h[1]], d = src[h[2]], f = src[h[3]];
+        Piece<V> o;
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          const float t = (bf2f(a.v[i]) + bf2f(b.v[i])) + (bf2f(d.v[i]) + bf2f(f.v[i]));
+          o.v[i] = f2bf(OP == 0 ? 0.25f * t : t);
+        }
+        dst[lo] = o;
+      } else {
+        Piece<V> o = src[lo];
+        if (OP == 1) {
+#pragma unroll
+          for (int i = 0; i < V; ++i) o.v[i] = f2bf(0.25f * bf2f(o.v[i]));
+        }
+        for (int i = 0; i < 4; ++i) dst[h[i]] = o;
+      }
+    }
+  }
+}
+
+// y[p] = (a[p], b[p]) (SPLIT false) or its adjoint (a[p], b[p]) = y[p]; pa, pb: pieces per pixel
+template <int V, bool SPLIT>
+__global__ void __launch_bounds__(256) nn_cat_k(bf16_t* __restrict__ a, unsigned pa, bf16_t* __restrict__ b, unsigned pb, long long n,
+                                                bf16_t* __restrict__ y) {
+  const unsigned pc = pa + pb;
   GS_LOOP(e, n) {
-    const int c = (int)(e % C);
-    const long long p = e / C;
-    const int X = (int)(p % Wo);
-    const long long t = p / Wo;
-    const int Y = (int)(t % Ho), b = (int)(t / Ho);
-    const long long base = (((long long)b * H + 2 * Y) * W + 2 * X) * C + c;
-    const float s = (bf2f(x[base]) + bf2f(x[base + C])) + (bf2f(x[base + (long long)W * C]) + bf2f(x[base + (long long)W * C + C]));
-    y[e] = f2bf(0.25f * s);
+    const long long p = n <= 0xffffffffLL ? (long long)((unsigned)e / pc) : e / pc;
+    const unsigned c = (unsigned)(e - p * pc);
+    Piece<V>* const o = c < pa ? (Piece<V>*)a + (p * pa + c) : (Piece<V>*)b + (p * pb + (c - pa));
+    if (SPLIT) *o = ((const Piece<V>*)y)[e];
+    else ((Piece<V>*)y)[e] = *o;
   }
 }
 
-__global__ void __launch_bounds__(256) nn_pool2_bwd_k(const bf16_t* __restrict__ dy, int B, int H, int W, int C, bf16_t* __restrict__ dx) {
-  const long long n = (long long)B * H * W * C;
-  GS_LOOP(e, n) {
-    const int c = (int)(e % C);
-    const long long p = e / C;
-    const int xx = (int)(p % W);
-    const long long t = p / W;
-    const int yy = (int)(t % H), b = (int)(t / H);
-    dx[e] = f2bf(0.25f * bf2f(dy[(((long long)b * (H / 2) + yy / 2) * (W / 2) + xx / 2) * C + c]));
-  }
-}
-
-__global__ void __launch_bounds__(256) nn_up2_k(const bf16_t* __restrict__ x, int B, int H, int W, int C, bf16_t* __restrict__ y) {
-  const int Ho = 2 * H, Wo = 2 * W;
-  const long long n = (long long)B * Ho * Wo * C;
-  GS_LOOP(e, n) {
-    const int c = (int)(e % C);
-    const long long p = e / C;
-    const int X = (int)(p % Wo);
-    const long long t = p / Wo;
-    const int Y = (int)(t % Ho), b = (int)(t / Ho);
-    y[e] = x[(((long long)b * H + Y / 2) * W + X / 2) * C + c];
-  }
-}
-
-__global__ void __launch_bounds__(256) nn_up2_bwd_k(const bf16_t* __restrict__ dy, int B, int H, int W, int C, bf16_t* __restrict__ dx) {
-  const long long n = (long long)B * H * W * C;
-  const int Wo = 2 * W;
-  GS_LOOP(e, n) {
-    const int c = (int)(e % C);
-    const long long p = e / C;
-    const int xx = (int)(p % W);
-    const long long t = p / W;
-    const int yy = (int)(t % H), b = (int)(t / H);
-    const long long base = (((long long)b * 2 * H + 2 * yy) * Wo + 2 * xx) * C + c;
-    const float s = (bf2f(dy[base]) + bf2f(dy[base + C])) + (bf2f(dy[base + (long long)Wo * C]) + bf2f(dy[base + (long long)Wo * C + C]));
-    dx[e] = f2bf(s);
-  }
-}
-
-__global__ void __launch_bounds__(256) nn_concat_k(const bf16_t* __restrict__ a, int Ca, const bf16_t* __restrict__ b, int Cb, long long P,
-                                                   bf16_t* __restrict__ y) {
-  const int C = Ca + Cb;
-  GS_LOOP(e, P * C) {
-    const int c = (int)(e % C);
-    const long long p = e / C;
-    y[e] = c < Ca ? a[p * Ca + c] : b[p * Cb + (c - Ca)];
-  }
-}
-
-__global__ void __launch_bounds__(256) nn_split_k(const bf16_t* __restrict__ dy, int Ca, int Cb, long long P, bf16_t* __restrict__ da,
-                                                  bf16_t* __restrict__ db) {
-  const int C = Ca + Cb;
-  GS_LOOP(e, P * C) {
-    const int c = (int)(e % C);
-    const long long p = e / C;
-    if (c < Ca) da[p * Ca + c] = dy[e];
-    else db[p * Cb + (c - Ca)] = dy[e];
-  }
-}
-
+template <int V>
 __global__ void __launch_bounds__(256) nn_relu_bwd_k(bf16_t* __restrict__ dy, const bf16_t* __restrict__ y, long long n) {
   GS_LOOP(e, n) {
-    if (!(bf2f(y[e]) > 0.f)) dy[e] = 0;
+    const Piece<V> a = ((const Piece<V>*)y)[e];
+    Piece<V> d = ((Piece<V>*)dy)[e];
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      if (!(bf2f(a.v[i]) > 0.f)) d.v[i] = 0;
+    ((Piece<V>*)dy)[e] = d;
   }
 }
 
-// db[n] += sum over rows of dy[m, n] (FP32); rows split over blockIdx.x in chunks of 256
-__global__ void __launch_bounds__(256) nn_bias_grad_k(const bf16_t* __restrict__ dy, long long M, int N, float* __restrict__ db) {
-  const long long r0 = (long long)blockIdx.x * 256, r1 = std::min<long long>(M, r0 + 256);
-  for (int n = threadIdx.x; n < N; n += 256) {
-    float s = 0.f;
-    for (long long m = r0; m < r1; ++m) s += bf2f(dy[m * N + n]);
-    atomicAdd(&db[n], s);
+// db[n] += sum over rows of dy[m, n] (FP32). Thread t of the T = (256 / units) * units that work sums
+// unit t % units (V channels) of every (T / units)-th row of the block's chunk; the partial sums of a
+// unit meet in LDS and go to db in one atomic per channel and block. (One thread per channel, as a
+// serial loop over 256 rows, took 24 to 60 us for the layers of a
+// training step of 8 x 128^2; this one 4.7 to 8.3.)
+template <int V>
+__global__ void __launch_bounds__(256) nn_bias_grad_k(const bf16_t* __restrict__ dy, long long M, int N, float* __restrict__ db, int chunk) {
+  __shared__ float part[256 * V];
+  const int units = N / V, u0 = blockIdx.y * 256, nu = min(256, units - u0), groups = 256 / nu, T = groups * nu;
+  const int t = threadIdx.x, u = t % nu, grp = t / nu;
+  const long long r0 = (long long)blockIdx.x * chunk, r1 = min(M, r0 + chunk);
+  float s[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) s[i] = 0.f;
+  if (t < T) {
+#pragma unroll 4
+    for (long long m = r0 + grp; m < r1; m += groups) {
+      const Piece<V> d = ((const Piece<V>*)dy)[m * units + u0 + u];
+#pragma unroll
+      for (int i = 0; i < V; ++i) s[i] += bf2f(d.v[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < V; ++i) part[t * V + i] = s[i];
+  __syncthreads();
+  for (int c = t; c < nu * V; c += 256) {
+    float v = 0.f;
+    for (int k = 0; k < groups; ++k) v += part[k * nu * V + c];
+    atomicAdd(&db[u0 * V + c], v);
   }
 }
 
@@ -595,8 +609,15 @@ __global__ void __launch_bounds__(256) nn_conv_flip_k(const bf16_t* __restrict__
     wf[e] = w[((long long)(8 - t) * Cin + ci) * Cout + co];
   }
 }
+template <int V>
 __global__ void __launch_bounds__(256) nn_add_bf16_k(bf16_t* __restrict__ y, const bf16_t* __restrict__ x, long long n) {
-  GS_LOOP(e, n) y[e] = f2bf(bf2f(y[e]) + bf2f(x[e]));
+  GS_LOOP(e, n) {
+    Piece<V> a = ((Piece<V>*)y)[e];
+    const Piece<V> b = ((const Piece<V>*)x)[e];
+#pragma unroll
+    for (int i = 0; i < V; ++i) a.v[i] = f2bf(bf2f(a.v[i]) + bf2f(b.v[i]));
+    ((Piece<V>*)y)[e] = a;
+  }
 }
 
 int launched(const char* what) {
@@ -772,44 +793,102 @@ extern "C" int ps_nn_col2im(const void* dcol, int B, int H, int W, int C, void* 
   NN_SIZES("ps_nn_col2im", B, H, W, C)
   NN_ELEMENTWISE(nn_col2im_k, (long long)B * H * W * C, (const bf16_t*)dcol, B, H, W, C, (bf16_t*)dx)
 }
+// 16-byte pieces of 8 elements: whole ones, on aligned pointers
+inline bool nn_pieces(std::initializer_list<long long> counts, std::initializer_list<const void*> ptrs) {
+  for (long long c : counts)
+    if (c % 8) return false;
+  for (const void* p : ptrs)
+    if ((uintptr_t)p & 15) return false;
+  return true;
+}
+
+namespace {
+// rows = B*H and W of the low-resolution image
+template <int OP>
+int quad_launch(const char* what, const void* in, long long rows, int W, int C, void* out, hipStream_t st) {
+  if (rows <= 0 || W <= 0 || C <= 0) return 0;
+  const bool v = nn_pieces({C}, {in, out});
+  const long long rp = (long long)W * (v ? C / 8 : C);
+  const dim3 grid((unsigned)std::min<long long>((rp + 255) / 256, 1 << 16), (unsigned)std::min<long long>(rows, 32768));
+  if (v) hipLaunchKernelGGL((nn_quad_k<OP, 8>), grid, dim3(256), 0, st, (const bf16_t*)in, rows, W, C, (bf16_t*)out);
+  else hipLaunchKernelGGL((nn_quad_k<OP, 1>), grid, dim3(256), 0, st, (const bf16_t*)in, rows, W, C, (bf16_t*)out);
+  return launched(what);
+}
+template <bool SPLIT>
+int cat_launch(const char* what, const void* a, int Ca, const void* b, int Cb, long long P, const void* y, hipStream_t st) {
+  if (P * ((long long)Ca + Cb) <= 0) return 0;
+  const bool v = nn_pieces({Ca, Cb}, {a, b, y});
+  const unsigned pa = v ? Ca / 8 : Ca, pb = v ? Cb / 8 : Cb;
+  const long long n = P * ((long long)pa + pb);
+  if (v) hipLaunchKernelGGL((nn_cat_k<8, SPLIT>), dim3(grid_for(n)), dim3(256), 0, st, (bf16_t*)a, pa, (bf16_t*)b, pb, n, (bf16_t*)y);
+  else hipLaunchKernelGGL((nn_cat_k<1, SPLIT>), dim3(grid_for(n)), dim3(256), 0, st, (bf16_t*)a, pa, (bf16_t*)b, pb, n, (bf16_t*)y);
+  return launched(what);
+}
+}  // namespace
+
+// whole pieces of 8 while n and the pointers allow it, else element by element
+#define NN_PIECEWISE(kernel, n, p, q)                                                                                        \
+  NN_BEGIN                                                                                                                   \
+  if ((n) <= 0) return 0;                                                                                                    \
+  if (nn_pieces({(long long)(n)}, {p, q}))                                                                                   \
+    hipLaunchKernelGGL((kernel<8>), dim3(grid_for((n) / 8)), dim3(256), 0, st, (bf16_t*)p, (const bf16_t*)q, (long long)(n) / 8); \
+  else                                                                                                                       \
+    hipLaunchKernelGGL((kernel<1>), dim3(grid_for(n)), dim3(256), 0, st, (bf16_t*)p, (const bf16_t*)q, (long long)(n));      \
+  return launched(#kernel);
+
 extern "C" int ps_nn_pool2(const void* x, int B, int H, int W, int C, void* y, void* stream) {
   NN_SIZES("ps_nn_pool2", B, H, W, C)
   if ((H | W) & 1) return ps_internal_fail(PS_EARGUMENT, "ps_nn_pool2: H and W must be even");
-  NN_ELEMENTWISE(nn_pool2_k, (long long)B * (H / 2) * (W / 2) * C, (const bf16_t*)x, B, H, W, C, (bf16_t*)y)
+  NN_BEGIN
+  return quad_launch<0>("ps_nn_pool2", x, (long long)B * (H / 2), W / 2, C, y, st);
 }
 extern "C" int ps_nn_pool2_bwd(const void* dy, int B, int H, int W, int C, void* dx, void* stream) {
   NN_SIZES("ps_nn_pool2_bwd", B, H, W, C)
   if ((H | W) & 1) return ps_internal_fail(PS_EARGUMENT, "ps_nn_pool2_bwd: H and W must be even");
-  NN_ELEMENTWISE(nn_pool2_bwd_k, (long long)B * H * W * C, (const bf16_t*)dy, B, H, W, C, (bf16_t*)dx)
+  NN_BEGIN
+  return quad_launch<1>("ps_nn_pool2_bwd", dy, (long long)B * (H / 2), W / 2, C, dx, st);
 }
 extern "C" int ps_nn_up2(const void* x, int B, int H, int W, int C, void* y, void* stream) {
   NN_SIZES("ps_nn_up2", B, H, W, C)
-  NN_ELEMENTWISE(nn_up2_k, (long long)B * 4 * H * W * C, (const bf16_t*)x, B, H, W, C, (bf16_t*)y)
+  NN_BEGIN
+  return quad_launch<2>("ps_nn_up2", x, (long long)B * H, W, C, y, st);
 }
 extern "C" int ps_nn_up2_bwd(const void* dy, int B, int H, int W, int C, void* dx, void* stream) {
   NN_SIZES("ps_nn_up2_bwd", B, H, W, C)
-  NN_ELEMENTWISE(nn_up2_bwd_k, (long long)B * H * W * C, (const bf16_t*)dy, B, H, W, C, (bf16_t*)dx)
+  NN_BEGIN
+  return quad_launch<3>("ps_nn_up2_bwd", dy, (long long)B * H, W, C, dx, st);
 }
 extern "C" int ps_nn_concat(const void* a, int Ca, const void* b, int Cb, int64_t P, void* y, void* stream) {
   NN_SIZES("ps_nn_concat", Ca, Cb, P)
-  NN_ELEMENTWISE(nn_concat_k, (long long)P * (Ca + Cb), (const bf16_t*)a, Ca, (const bf16_t*)b, Cb, (long long)P, (bf16_t*)y)
+  NN_BEGIN
+  return cat_launch<false>("ps_nn_concat", a, Ca, b, Cb, P, y, st);
 }
 extern "C" int ps_nn_split(const void* dy, int Ca, int Cb, int64_t P, void* da, void* db, void* stream) {
   NN_SIZES("ps_nn_split", Ca, Cb, P)
-  NN_ELEMENTWISE(nn_split_k, (long long)P * (Ca + Cb), (const bf16_t*)dy, Ca, Cb, (long long)P, (bf16_t*)da, (bf16_t*)db)
+  NN_BEGIN
+  return cat_launch<true>("ps_nn_split", da, Ca, db, Cb, P, dy, st);
 }
-extern "C" int ps_nn_relu_bwd(void* dy, const void* y, int64_t n, void* stream) {
-  NN_ELEMENTWISE(nn_relu_bwd_k, (long long)n, (bf16_t*)dy, (const bf16_t*)y, (long long)n)
-}
+extern "C" int ps_nn_relu_bwd(void* dy, const void* y, int64_t n, void* stream) { NN_PIECEWISE(nn_relu_bwd_k, n, dy, y) }
 extern "C" int ps_nn_bias_grad(const void* dy, int64_t M, int N, float* db, void* stream) {
   NN_BEGIN
   if (M <= 0 || N <= 0) return 0;
-  hipLaunchKernelGGL(nn_bias_grad_k, dim3((unsigned)((M + 255) / 256)), dim3(256), 0, st, (const bf16_t*)dy, (long long)M, N, db);
+  const bool v = nn_pieces({N}, {dy});
+  const int units = v ? N / 8 : N;
+  // about one workgroup per CU, at least 64 rows each: one atomic per channel and workgroup
+  const int chunk = (int)std::min<long long>(std::max<long long>(64, (M + 255) / 256), 1 << 30);
+  const dim3 grid((unsigned)((M + chunk - 1) / chunk), (unsigned)((units + 255) / 256));
+  if (v) hipLaunchKernelGGL((nn_bias_grad_k<8>), grid, dim3(256), 0, st, (const bf16_t*)dy, (long long)M, N, db, chunk);
+  else hipLaunchKernelGGL((nn_bias_grad_k<1>), grid, dim3(256), 0, st, (const bf16_t*)dy, (long long)M, N, db, chunk);
   return launched("ps_nn_bias_grad");
 }
 extern "C" int ps_nn_mse(const void* pred, const float* target, const float* mask, int64_t n, float scale, void* dpred, float* loss,
                          void* stream) {
-  NN_ELEMENTWISE(nn_mse_k, (long long)n, (const bf16_t*)pred, target, mask, (long long)n, scale, (bf16_t*)dpred, loss)
+  NN_BEGIN
+  if (n <= 0) return 0;
+  // every workgroup ends in one atomic on the loss: a few hundred of them at most (1536 took 22 us)
+  hipLaunchKernelGGL(nn_mse_k, dim3(std::min(grid_for(n), 256u)), dim3(256), 0, st, (const bf16_t*)pred, target, mask, (long long)n, scale,
+                     (bf16_t*)dpred, loss);
+  return launched("ps_nn_mse");
 }
 extern "C" int ps_nn_adam(float* w, const float* g, float* m, float* v, int64_t n, float lr, float b1, float b2, float eps, float c1, float c2,
                           void* w16, void* stream) {
@@ -822,9 +901,7 @@ extern "C" int ps_nn_bf16_to_f32(const void* x, int64_t n, float* y, void* strea
   NN_ELEMENTWISE(nn_bf16_to_f32_k, (long long)n, (const bf16_t*)x, (long long)n, y)
 }
 extern "C" int ps_nn_fill_f32(float* x, int64_t n, float v, void* stream) { NN_ELEMENTWISE(nn_fill_f32_k, (long long)n, x, (long long)n, v) }
-extern "C" int ps_nn_add_bf16(void* y, const void* x, int64_t n, void* stream) {
-  NN_ELEMENTWISE(nn_add_bf16_k, (long long)n, (bf16_t*)y, (const bf16_t*)x, (long long)n)
-}
+extern "C" int ps_nn_add_bf16(void* y, const void* x, int64_t n, void* stream) { NN_PIECEWISE(nn_add_bf16_k, n, y, x) }
 
 extern "C" int ps_nn_alloc(int64_t bytes, void** out) {
   if (int r = ps_internal_require_init()) return r;
