@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <string>
+#include <type_traits>
 
 #include "ps_amd.h"
 #include "ps_internal.h"
@@ -411,6 +412,139 @@ __global__ void __launch_bounds__(64 * WM * WN) nn_conv3_k(const bf16_t* __restr
   }
 }
 
+// ---- weight gradient of a 3x3 convolution: gw[tap*C + c][n] += sum over pixels x(pixel + tap, c) dy(pixel, n)
+//
+// A workgroup sums a share of the pixel tiles (256 pixels: TX columns wide) for 32 input channels x 32
+// output channels x all nine taps: the patch of x and the tile of dy are read from memory once and
+// held in LDS as [pixel][channel], the next tile's loads in flight meanwhile. Both MFMA operands need
+// 8 consecutive pixels of one channel per lane, which the transposing LDS read takes out of
+// [pixel][channel] at any shift. Wavefront w of each half multiplies every fourth group of 32 pixels by
+// 16 of the input channels into its own 9 x 2 accumulators (all 32 in one wavefront spilled); they
+// are summed in LDS and added to gw with one atomic per element and workgroup. The general product read x nine times, split K over hundreds of
+// workgroups of one 64 x 64 tile each, and spent 32 of its 64 columns on padding.
+constexpr int WGS = 40;  // LDS elements per pixel: 32 channels, 16 bytes of padding against bank conflicts
+
+template <bool VEC>
+__global__ void __launch_bounds__(512, 2) nn_conv3_wgrad_k(const bf16_t* __restrict__ x, int H, int W, int C, const bf16_t* __restrict__ dy,
+                                                           long long sbk, int N, float* __restrict__ gw, long long ldc, int lgTX, int tilesx,
+                                                           int tilesy, int ntiles, unsigned pmagic) {
+  __shared__ __attribute__((aligned(16))) bf16_t lds[(340 + 256) * WGS];
+  constexpr int RS = 36;  // row stride of the FP32 sums [4 wavefronts][2 taps][32][RS]
+  static_assert(4 * 2 * 32 * RS * 4 <= (int)sizeof(lds), "the sums reuse the tiles' memory");
+  bf16_t* const xs = lds;
+  bf16_t* const ds = lds + 340 * WGS;
+  const int TX = 1 << lgTX, PW = TX + 2, rows = 256 >> lgTX, npx = (rows + 2) * PW;  // at most 340 patch pixels
+  const int tid = threadIdx.x, lane = tid & 63, w = (tid >> 6) & 3, ct = tid >> 8, g = lane >> 4, li = lane & 15;
+  const int c0 = blockIdx.x * 32, n0 = blockIdx.y * 32;
+  s16x8 rx[3], rd[2];
+  auto load = [&](int t) {
+    const int tx0 = (t % tilesx) << lgTX, t2 = t / tilesx, ty0 = (t2 % tilesy) * rows, img = t2 / tilesy;
+    const long long pb = (long long)img * H * W;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const unsigned e = tid + 512 * j, p = e >> 2, py = __umulhi(p, pmagic);
+      const int yy = ty0 + (int)py - 1, xx = tx0 + (int)(p - py * PW) - 1, c = c0 + 8 * (int)(e & 3);
+      rx[j] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (p < (unsigned)npx && (unsigned)yy < (unsigned)H && (unsigned)xx < (unsigned)W) {
+        const bf16_t* const src = x + (pb + (long long)yy * W + xx) * C + c;
+        if (VEC) {
+          if (c < C) rx[j] = *(const s16x8*)src;
+        } else {
+          for (int i = 0; i < 8; ++i)
+            if (c + i < C) rx[j][i] = (short)src[i];
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int e = tid + 512 * j, p = e >> 2, yy = ty0 + (p >> lgTX), xx = tx0 + (p & (TX - 1)), n = n0 + 8 * (e & 3);
+      rd[j] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (yy < H && xx < W) {
+        const bf16_t* const src = dy + (pb + (long long)yy * W + xx) * sbk + n;
+        if (VEC) {
+          if (n < N) rd[j] = *(const s16x8*)src;
+        } else {
+          for (int i = 0; i < 8; ++i)
+            if (n + i < N) rd[j][i] = (short)src[i];
+        }
+      }
+    }
+  };
+  f32x4 acc[9][2];
+#pragma unroll
+  for (int a = 0; a < 9; ++a)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[a][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int t = blockIdx.z;
+  load(t);
+  while (t < ntiles) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int e = tid + 512 * j;
+      if ((e >> 2) < npx) *(s16x8*)&xs[(e >> 2) * WGS + 8 * (e & 3)] = rx[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int e = tid + 512 * j;
+      *(s16x8*)&ds[(e >> 2) * WGS + 8 * (e & 3)] = rd[j];
+    }
+    __syncthreads();
+    const int tx0 = (t % tilesx) << lgTX, ty0 = ((t / tilesx) % tilesy) * rows;
+    t += gridDim.z;
+    if (t < ntiles) load(t);
+    auto products = [&](auto masked) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int q0 = (w + 4 * h) * 32 + 8 * g, q = q0 + (li >> 2), row = q >> lgTX, col = q & (TX - 1);
+        s16x8 b[2], keep;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          b[j] = cat8(lds_tr(&ds[q * WGS + 16 * j + 4 * (li & 3)]), lds_tr(&ds[(q + 4) * WGS + 16 * j + 4 * (li & 3)]));
+        if (masked) {
+          const int left = ty0 + (q0 >> lgTX) < H ? W - tx0 - (q0 & (TX - 1)) : 0;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) keep[i] = i < left ? (short)-1 : (short)0;
+        }
+        const bf16_t* const xp = &xs[(row * PW + col) * WGS + 16 * ct + 4 * (li & 3)];
+#pragma unroll
+        for (int a = 0; a < 9; ++a) {
+          const bf16_t* const xa = xp + ((a / 3) * PW + a % 3) * WGS;
+          s16x8 v = cat8(lds_tr(xa), lds_tr(xa + 4 * WGS));
+          if (masked) v &= keep;
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[a][j] = mfma(v, b[j], acc[a][j]);
+        }
+      }
+    };
+    // pixels outside the image take no part (an infinite x there would make a NaN of its zero dy)
+    if (tx0 + TX > W || ty0 + rows > H) products(std::true_type{});
+    else products(std::false_type{});
+    __syncthreads();
+  }
+  // the four wavefronts' sums meet in LDS, two taps at a time (LDS atomics took 60 us here, one
+  // wavefront after the other 25)
+  float* const red = (float*)lds;
+#pragma unroll
+  for (int a0 = 0; a0 < 9; a0 += 2) {
+#pragma unroll
+    for (int a = a0; a < a0 + 2 && a < 9; ++a)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[((w * 2 + a - a0) * 32 + 16 * ct + 4 * g + r) * RS + 16 * j + li] = acc[a][j][r];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int e = tid + 512 * k, n = e & 31, c = (e >> 5) & 31, a = e >> 10;
+      if (a0 + a < 9 && c0 + c < C && n0 + n < N) {
+        const float* const p = &red[(a * 32 + c) * RS + n];
+        unsafeAtomicAdd(&gw[(long long)((a0 + a) * C + c0 + c) * ldc + n0 + n], (p[0] + p[2 * 32 * RS]) + (p[4 * 32 * RS] + p[6 * 32 * RS]));
+      }
+    }
+    __syncthreads();
+  }
+}
+
 unsigned grid_for(long long n) { return (unsigned)std::min<long long>((n + 255) / 256, 1 << 20); }
 
 #define GS_LOOP(e, n) for (long long e = (long long)blockIdx.x * 256 + threadIdx.x; e < (n); e += (long long)gridDim.x * 256)
@@ -742,6 +876,34 @@ int conv3_launch(int M, int N, const bf16_t* x, int H, int W, int C, const bf16_
   return launched("ps_nn_gemm_im2col");
 }
 
+// The weight gradient by nn_conv3_wgrad_k, or 1 where the general product serves: a single K chain
+// (splitk 1) keeps its order of summation.
+int wgrad_launch(int N, long long K, const bf16_t* x, int H, int W, int C, const bf16_t* dy, long long sbk, long long sbn, void* gw, long long ldc, int epi,
+                 int splitk, hipStream_t st) {
+  if (splitk < 2 || epi != PS_NN_EPI_F32_ADD || sbn != 1) return 1;
+  const long long imgs = K / ((long long)H * W);
+  auto up = [](long long a, long long b) { return (a + b - 1) / b; };
+  // the tile width (32, 16 or 8 pixels of 256) that pads the images least
+  int lg = 5;
+  long long best = up(W, 32) * up(H, 8);
+  for (int l : {4, 3})
+    if (up(W, 1 << l) * up(H, 256 >> l) < best) best = up(W, 1 << l) * up(H, 256 >> l), lg = l;
+  const int tx = 1 << lg, tilesx = (int)up(W, tx), tilesy = (int)up(H, 256 >> lg);
+  const long long nt = best * imgs, gc = up(C, 32), gn = up(N, 32);
+  if (nt > 0x7fffffffLL || gn > 65535) return 1;
+  // A workgroup ends in 9216 atomics: about 128 workgroups of at least four tiles, 256 from 1024 tiles
+  // on (8 x 128^2, 32 -> 32, 512 tiles: 15.3 us with 128 workgroups, 18.1 with 256, 28.8 with 512;
+  // 96 -> 32, 1536 tiles: 27.2, 22.7, 30.6; 8 x 32^2, 384 -> 128: 32.7, 19.8, 26.1)
+  const long long want = nt * gc * gn < 1024 ? 128 : 256;
+  const int S = (int)std::min<long long>(std::min<long long>(nt, 65535), std::max<long long>(1, want / (gc * gn)));
+  const unsigned pmagic = (unsigned)((0x100000000ULL + tx + 1) / (tx + 2));
+  const dim3 grid((unsigned)gc, (unsigned)gn, (unsigned)S);
+  const bool v = C % 8 == 0 && N % 8 == 0 && sbk % 8 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)dy & 15) == 0;
+  if (v) hipLaunchKernelGGL((nn_conv3_wgrad_k<true>), grid, dim3(512), 0, st, x, H, W, C, dy, sbk, N, (float*)gw, ldc, lg, tilesx, tilesy, (int)nt, pmagic);
+  else hipLaunchKernelGGL((nn_conv3_wgrad_k<false>), grid, dim3(512), 0, st, x, H, W, C, dy, sbk, N, (float*)gw, ldc, lg, tilesx, tilesy, (int)nt, pmagic);
+  return launched("ps_nn_gemm_im2col");
+}
+
 }  // namespace
 
 extern "C" int ps_nn_gemm(int M, int N, int K, const void* A, int64_t sam, int64_t sak, const void* B, int64_t sbk, int64_t sbn, void* C,
@@ -759,6 +921,10 @@ extern "C" int ps_nn_gemm_im2col(int transpose, int M, int N, int K, const void*
     return ps_internal_fail(PS_EARGUMENT, "ps_nn_gemm_im2col: the im2col operand is (B*H*W) x (9*C): sizes do not match");
   if (!transpose && M > 0 && N > 0 && (epi == PS_NN_EPI_BF16 || bias)) {
     const int r = conv3_launch(M, N, (const bf16_t*)x, H, W, Cin, (const bf16_t*)B, sbk, sbn, C, ldc, bias, epi, splitk, st);
+    if (r <= 0) return r;
+  }
+  if (transpose && M > 0 && N > 0 && K > 0) {
+    const int r = wgrad_launch(N, K, (const bf16_t*)x, H, W, Cin, (const bf16_t*)B, sbk, sbn, C, ldc, epi, splitk, st);
     if (r <= 0) return r;
   }
   return transpose ? gemm_launch<2>(M, N, K, x, 0, 0, B, sbk, sbn, C, ldc, bias, epi, splitk, st, H, W, Cin)
