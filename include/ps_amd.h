@@ -250,6 +250,30 @@ int ps_field_reduce(const ps_field* f, int op, double* out, void* stream);
  * nothing to the host and does not wait, so it can be captured into a graph. More than 4 fields
  * fail with PS_EARGUMENT. Calls that overlap on one GPU share that array and race. */
 int ps_field_reduce_noalloc(const ps_field* fields, int nfields, int op, double* out, void* stream);
+/* No counterpart in the reference: ps_field_reduce_noalloc of every z plane by itself, for 1..4 fields of
+ * the same number of planes: out[s*nfields + i] (device memory) receives the statistic of plane s of
+ * fields[i], in the order of summation of a 2-D field. The partial sums go to work, nwork doubles of
+ * device memory of the caller's: at least 4*min(ceil(nx*ny/256), 2048) (the largest field's) times
+ * planes times nfields. */
+int ps_plane_reduce_noalloc(const ps_field* fields, int nfields, int op, double* work, int64_t nwork, double* out, void* stream);
+
+/* n pseudo-time iterations of the Stokes2D solver (miniapps/Stokes2D.jl:111-116: compute_P!, compute_τ!,
+ * compute_dV!, compute_V! and the free-slip copies) on S samples, several iterations per launch,
+ * asynchronous on `stream` and capturable. Replaces n times the launches of those kernels: the fields
+ * afterwards are bit for bit theirs. All fields are FP64 of one problem of nx x ny cells, (.., .., S):
+ * state and alt {Vx, Vy, Pt, dVxdτ, dVydτ} (alt: scratch of the same sizes, contents undefined), coef
+ * {dτPt, Mus, dτVx, dτVy, Rog}, out {∇V, τxx, τyy, τxy, Rx, Ry} (those of the last iteration). act with a
+ * device pointer: one flag per sample at act.ptr + s*act.plane, 0 leaves all fields of that sample as
+ * they are; act.ptr NULL: all iterate. n is 0 or at least 2; 8 to 32768 cells per dimension. */
+typedef struct ps_stokes2d {
+  ps_field state[5];
+  ps_field alt[5];
+  ps_field coef[5];
+  ps_field out[6];
+  ps_field act;
+  double dx, dy, dampX, dampY;
+} ps_stokes2d;
+int ps_stokes2d_iterate(const ps_stokes2d* problem, int n, void* stream);
 
 /* ---- events (measurement; no reference counterpart: the reference times with
  * wall-clock T_eff prints, README.md:457-464) ---- */

@@ -142,6 +142,20 @@ class ps_devinfo(ctypes.Structure):
     ]
 
 
+class ps_stokes2d(ctypes.Structure):
+    _fields_ = [
+        ("state", ps_field * 5),
+        ("alt", ps_field * 5),
+        ("coef", ps_field * 5),
+        ("out", ps_field * 6),
+        ("act", ps_field),
+        ("dx", ctypes.c_double),
+        ("dy", ctypes.c_double),
+        ("dampX", ctypes.c_double),
+        ("dampY", ctypes.c_double),
+    ]
+
+
 # name -> (restype, argtypes); every function returns int status unless noted
 _P = ctypes.POINTER
 _SIGS = {
@@ -161,6 +175,9 @@ _SIGS = {
     "ps_field_copy": (ctypes.c_int, [_P(ps_field), _P(ps_field), ctypes.c_void_p]),
     "ps_field_reduce": (ctypes.c_int, [_P(ps_field), ctypes.c_int, _P(ctypes.c_double), ctypes.c_void_p]),
     "ps_field_reduce_noalloc": (ctypes.c_int, [_P(ps_field), ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]),
+    "ps_plane_reduce_noalloc": (ctypes.c_int, [_P(ps_field), ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+                                               ctypes.c_void_p]),
+    "ps_stokes2d_iterate": (ctypes.c_int, [_P(ps_stokes2d), ctypes.c_int, ctypes.c_void_p]),
     "ps_stream_get": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _P(ctypes.c_void_p)]),
     "ps_stream_sync": (ctypes.c_int, [ctypes.c_void_p]),
     "ps_kernel_define": (ctypes.c_int, [ctypes.c_char_p, ctypes.c_char_p, _P(ctypes.c_void_p)]),

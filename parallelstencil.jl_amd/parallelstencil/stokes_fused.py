@@ -28,7 +28,7 @@ import re
 import numpy as np
 
 from . import core
-from ._lib import check, lib
+from ._lib import check, lib, ps_stokes2d
 from . import workloads as W
 
 STOKES2D_PTAU = """
@@ -86,6 +86,32 @@ end
 """
 
 
+class _Iterations:
+    """ps_stokes2d_iterate on a solver's fields: several PT iterations per launch. The launches read
+    the state from one copy and write the other, so a second copy of the five state arrays is held."""
+
+    MIN = 8  # cells per dimension
+
+    def __init__(self, sv, act=None):
+        self.fields = dict(state=(sv.Vx, sv.Vy, sv.Pt, sv.dVxdt, sv.dVydt), coef=(sv.dtPt, sv.Mus, sv.dtVx, sv.dtVy, sv.Rog),
+                           out=(sv.divV, sv.txx, sv.tyy, sv.txy, sv.Rx, sv.Ry))
+        self.fields["alt"] = tuple(core.zeros(*A.shape, eltype=core.Float64) for A in self.fields["state"])
+        self.act = act
+        self.q = ps_stokes2d(dx=sv.dx, dy=sv.dy, dampX=sv.dampX, dampY=sv.dampY)
+        self.stream = core._stream_handle(None)
+
+    def __call__(self, n):
+        for name, arrs in self.fields.items():
+            dst = getattr(self.q, name)
+            for i, A in enumerate(arrs):
+                if not A._alive():
+                    raise core.ArgumentError("an array of this solver has been freed")
+                dst[i] = A.f
+        if self.act is not None:
+            self.q.act = self.act.f
+        check(lib.ps_stokes2d_iterate(ctypes.byref(self.q), n, self.stream))
+
+
 class Stokes2DFused:
     """miniapps/Stokes2D.jl:62-125 with two launches per PT iteration (module docstring). Same
     interface as workloads.Stokes2D: set_material, reset, iterate, iterate_block, error, solve."""
@@ -123,6 +149,7 @@ class Stokes2DFused:
             self.k_dvv.launcher(self.Rx, self.Ry, self.dVxdt, self.dVydt, self.Vx, self.Vy, self.Pt, self.Rog, self.txx, self.tyy,
                                 self.txy, self.dtVx, self.dtVy, self.dampX, self.dampY, self.dx, self.dy, ranges=rng),
         ]
+        self._many = _Iterations(self) if min(nx, ny) >= _Iterations.MIN else None
         self._graph = None
         self._host_err = np.zeros(4)
         self.iterate(1)  # compiles and loads both kernels (zero fields stay zero)
@@ -154,7 +181,11 @@ class Stokes2DFused:
             self.Pt.copy_from(Pt)
 
     def iterate(self, n):
-        """n PT iterations (miniapps/Stokes2D.jl:111-116), asynchronous."""
+        """n PT iterations (miniapps/Stokes2D.jl:111-116), asynchronous: several per launch, a single
+        one by the two kernels above."""
+        if n > 1 and self._many is not None:
+            self._many(n)
+            return
         a, b = self._steps
         for _ in range(n):
             a()
@@ -282,13 +313,10 @@ class Stokes2DBatch:
         self.dVxdt, self.dVydt = z(nx - 1, ny - 2), z(nx - 2, ny - 1)
         self.dtVx, self.dtVy = z(nx - 1, ny - 2), z(nx - 2, ny - 1)
         self.Mus, self.Rog, self.Mts, self.Mtmp = z(nx, ny), z(nx, ny), z(nx, ny), z(nx, ny)
-        # the residual check: mean |Rx|, mean |Ry|, mean |∇V| of every sample's plane, reduced in
-        # calls of at most 4 plane views (one stream, so the calls never overlap)
-        planes = [A.view((1, 1, s), (A.shape[0], A.shape[1], s)) for s in range(1, S + 1) for A in (self.Rx, self.Ry, self.divV)]
-        self._planes = planes  # the views hold their parents
-        self.err_d = core.zeros(4 * ((3 * S + 3) // 4), eltype=core.Float64)
-        self._red = [((core.ps_field * len(planes[c:c + 4]))(*[v.f for v in planes[c:c + 4]]), len(planes[c:c + 4]), self.err_d.ptr + 8 * c)
-                     for c in range(0, 3 * S, 4)]
+        # the residual check: mean |Rx|, mean |Ry|, mean |∇V| of every sample's plane
+        self.err_d = core.zeros(3 * S, eltype=core.Float64)
+        self._red = (core.ps_field * 3)(self.Rx.f, self.Ry.f, self.divV.f)
+        self._red_work = core.zeros(4 * min(-(-nx * ny // 256), 2048) * 3 * S, eltype=core.Float64)
         rng = ((1, nx), (1, ny), (1, S))
         self._rng = rng
         self._steps = [
@@ -297,6 +325,7 @@ class Stokes2DBatch:
             self.k_dvv.launcher(self.Act, self.Rx, self.Ry, self.dVxdt, self.dVydt, self.Vx, self.Vy, self.Pt, self.Rog, self.txx,
                                 self.tyy, self.txy, self.dtVx, self.dtVy, self.dampX, self.dampY, self.dx, self.dy, ranges=rng),
         ]
+        self._many = _Iterations(self, self.Act) if min(nx, ny) >= _Iterations.MIN else None
         self._graph = None
         self.iterate(1)  # compiles and loads both kernels (no plane is active yet)
         self._check()
@@ -334,14 +363,17 @@ class Stokes2DBatch:
 
     def iterate(self, n):
         """n PT iterations of every sample, asynchronous."""
+        if n > 1 and self._many is not None:
+            self._many(n)
+            return
         a, b = self._steps
         for _ in range(n):
             a()
             b()
 
     def _check(self):
-        for fields, n, out in self._red:
-            check(lib.ps_field_reduce_noalloc(fields, n, 3, ctypes.c_void_p(out), None))
+        check(lib.ps_plane_reduce_noalloc(self._red, 3, 3, ctypes.c_void_p(self._red_work.ptr), len(self._red_work),
+                                          ctypes.c_void_p(self.err_d.ptr), None))
 
     def iterate_block(self):
         """nout iterations and the residual reductions: one graph replay (captured on first use)."""

@@ -1,0 +1,150 @@
+"""The tiled network kernels at the sizes where their tiles, masks and dispatch rules change: the 3x3
+convolution and its weight gradient against the stored column matrix, the piecewise data movement
+against one element at a time (a pointer shifted by one element takes that path), the bias gradient
+against float64 sums."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import parallelstencil as ps
+from parallelstencil import unet as U
+from parallelstencil._lib import lib
+
+pytestmark = pytest.mark.gpu
+ps.ensure_device()
+
+
+def _bf(a):
+    return ps.bf16_to_f32(ps.f32_to_bf16(np.asarray(a, np.float32)))
+
+
+# image sizes around the 8- and 16-column tiles, channels around the groups of 8 and 32 and beyond what
+# fits two patches (and one patch) into LDS, output channels around 32 and 64
+CONV = [(1, 1, 1, 8, 8), (2, 15, 17, 32, 33), (1, 16, 16, 24, 31), (3, 9, 8, 40, 65), (1, 33, 31, 7, 4), (2, 20, 24, 128, 130), (1, 70, 70, 96, 32),
+        (4, 64, 64, 192, 64), (1, 10, 40, 384, 96), (1, 12, 12, 512, 16), (1, 300, 260, 32, 32), (2, 5, 100, 9, 12), (1, 17, 130, 2, 3)]
+
+
+@pytest.mark.parametrize("B,H,W,C,N", CONV)
+def test_convolution_matches_the_column_matrix(B, H, W, C, N):
+    rng = np.random.default_rng(B * H * W + C + N)
+    P, K = B * H * W, 9 * C
+    x, w = U.Buf((B, H, W, C)).upload(rng.standard_normal((B, H, W, C))), U.Buf((K, N)).upload(rng.standard_normal((K, N)))
+    bias, col = U.Buf((N,), "f32").upload(rng.standard_normal(N)), U.Buf((P, K))
+    ps.core.check(lib.ps_nn_im2col(x.p, B, H, W, C, col.p, None))
+    for epi in (U.EPI_BF16, U.EPI_BIAS, U.EPI_BIAS_RELU):
+        ye, yi = U.Buf((P, N)), U.Buf((P, N))
+        U.gemm(P, N, K, col, K, 1, w, N, 1, ye, N, bias, epi)
+        U.gemm_im2col(0, P, N, K, x, H, W, C, w, N, 1, yi, N, bias, epi)
+        assert np.array_equal(ye.download(), yi.download()), epi
+
+
+@pytest.mark.parametrize("strides", ["transposed", "wide"])
+def test_convolution_with_other_weight_and_result_strides(strides):
+    rng = np.random.default_rng(3)
+    B, H, W, C, N = 1, 20, 20, 32, 40
+    P, K = B * H * W, 9 * C
+    x, wh = U.Buf((B, H, W, C)).upload(rng.standard_normal((B, H, W, C))), _bf(rng.standard_normal((K, N)))
+    col = U.Buf((P, K))
+    ps.core.check(lib.ps_nn_im2col(x.p, B, H, W, C, col.p, None))
+    if strides == "transposed":
+        w, sk, sn, ld = U.Buf((N, K)).upload(wh.T), 1, K, N
+    else:
+        w, sk, sn, ld = U.Buf((K, N + 3)).upload(np.pad(wh, ((0, 0), (0, 3)))), N + 3, 1, N + 5
+    ye, yi = U.Buf((P, ld)), U.Buf((P, ld))
+    U.gemm(P, N, K, col, K, 1, w, sk, sn, ye, ld)
+    U.gemm_im2col(0, P, N, K, x, H, W, C, w, sk, sn, yi, ld)
+    assert np.array_equal(ye.download(), yi.download())
+
+
+@pytest.mark.parametrize("special", [np.inf, np.nan])
+def test_convolution_of_infinities_and_nan(special):
+    # a value outside the window of a pixel, or behind the last k, must not reach it
+    rng = np.random.default_rng(5)
+    B, H, W, C, N = 1, 18, 21, 24, 40
+    P, K = B * H * W, 9 * C
+    xh = rng.standard_normal((B, H, W, C))
+    xh[0, 7, 9, 3] = special
+    x, w, col = U.Buf(xh.shape).upload(xh), U.Buf((K, N)).upload(rng.standard_normal((K, N))), U.Buf((P, K))
+    ps.core.check(lib.ps_nn_im2col(x.p, B, H, W, C, col.p, None))
+    ye, yi = U.Buf((P, N)), U.Buf((P, N))
+    U.gemm(P, N, K, col, K, 1, w, N, 1, ye, N)
+    U.gemm_im2col(0, P, N, K, x, H, W, C, w, N, 1, yi, N)
+    a, b = ye.download(), yi.download()
+    assert np.array_equal(a, b, equal_nan=True) and np.isfinite(b).sum() == (P - 9) * N
+    dy = U.Buf((P, N)).upload(rng.standard_normal((P, N)))
+    ge, gi = U.Buf((K, N), "f32").zero(), U.Buf((K, N), "f32").zero()
+    U.gemm(K, N, P, col, 1, K, dy, N, 1, ge, N, epi=U.EPI_F32_ADD, splitk=2)
+    U.gemm_im2col(1, K, N, P, x, H, W, C, dy, N, 1, gi, N, epi=U.EPI_F32_ADD, splitk=2)
+    assert np.array_equal(np.isfinite(ge.download()), np.isfinite(gi.download()))
+
+
+@pytest.mark.parametrize("B,H,W,C,N", CONV)
+def test_weight_gradient_against_float64(B, H, W, C, N):
+    """FP32 sums of P products of BF16 values in any order: within P eps of the sum of magnitudes in
+    the worst case; sqrt(P) growth with a factor 8 is far inside it and far above what is seen."""
+    rng = np.random.default_rng(B + H + W + C + N)
+    P, K = B * H * W, 9 * C
+    xh, dh = _bf(rng.standard_normal((B, H, W, C))), _bf(rng.standard_normal((P, N)))
+    x, dy = U.Buf(xh.shape).upload(xh), U.Buf(dh.shape).upload(dh)
+    g = U.Buf((K, N), "f32").upload(np.ones((K, N)))
+    U.gemm_im2col(1, K, N, P, x, H, W, C, dy, N, 1, g, N, epi=U.EPI_F32_ADD, splitk=2)
+    xp = np.pad(xh.astype(np.float64), ((0, 0), (1, 1), (1, 1), (0, 0)))
+    d64 = dh.astype(np.float64)
+    got = g.download().astype(np.float64) - 1.0
+    for t in range(9):
+        ref = xp[:, t // 3:t // 3 + H, t % 3:t % 3 + W].reshape(P, C).T @ d64
+        assert np.abs(got[t * C:(t + 1) * C] - ref).max() <= 8 * 2.0 ** -24 * (P + 4 * np.sqrt(P)), t
+
+
+def _shifted(a, off):
+    """A device copy of `a` that starts `off` elements into its buffer."""
+    b = U.Buf((a.size + 8,))
+    b.upload(np.concatenate([np.zeros(off), a.reshape(-1), np.zeros(8 - off)]))
+    return b, ctypes.c_void_p(b.p.value + 2 * off)
+
+
+def _read(b, off, n):
+    return b.download()[off:off + n]
+
+
+@pytest.mark.parametrize("C", [8, 24, 64, 5])
+def test_data_movement_in_pieces_matches_single_elements(C):
+    rng = np.random.default_rng(C)
+    B, H, W = 2, 6, 10
+    lo, hi = rng.standard_normal((B, H, W, C)), rng.standard_normal((B, 2 * H, 2 * W, C))
+    for name, src, n, args in (("ps_nn_up2", lo, hi.size, (B, H, W, C)), ("ps_nn_up2_bwd", hi, lo.size, (B, H, W, C)),
+                               ("ps_nn_pool2", hi, lo.size, (B, 2 * H, 2 * W, C)), ("ps_nn_pool2_bwd", lo, hi.size, (B, 2 * H, 2 * W, C))):
+        outs = []
+        for off in (0, 1):
+            (s, sp), (d, dp) = _shifted(src, off), _shifted(np.zeros(n), off)
+            ps.core.check(getattr(lib, name)(sp, *args, dp, None))
+            outs.append(_read(d, off, n))
+        assert np.array_equal(*outs) and np.any(outs[0]), name
+    P, Cb = B * H * W, 16 if C % 8 == 0 else 3
+    a, b = rng.standard_normal((P, C)), rng.standard_normal((P, Cb))
+    for off in (0, 1):
+        (_a, ap), (_b, bp), (y, yp) = _shifted(a, off), _shifted(b, off), _shifted(np.zeros((P, C + Cb)), off)
+        ps.core.check(lib.ps_nn_concat(ap, C, bp, Cb, P, yp, None))
+        assert np.array_equal(_read(y, off, P * (C + Cb)).reshape(P, -1), np.concatenate([_bf(a), _bf(b)], 1))
+        (da, dap), (db, dbp) = _shifted(0 * a, off), _shifted(0 * b, off)
+        ps.core.check(lib.ps_nn_split(yp, C, Cb, P, dap, dbp, None))
+        assert np.array_equal(_read(da, off, a.size), _bf(a).reshape(-1)) and np.array_equal(_read(db, off, b.size), _bf(b).reshape(-1))
+    n = P * C
+    for off in (0, 1):
+        (d, dp), (y, yp) = _shifted(a, off), _shifted(lo, off)
+        ps.core.check(lib.ps_nn_relu_bwd(dp, yp, n, None))
+        assert np.array_equal(_read(d, off, n), np.where(_bf(lo).reshape(-1) > 0, _bf(a).reshape(-1), 0))
+        ps.core.check(lib.ps_nn_add_bf16(dp, yp, n, None))
+        want = _bf(np.where(_bf(lo).reshape(-1) > 0, _bf(a).reshape(-1), 0) + _bf(lo).reshape(-1))
+        assert np.array_equal(_read(d, off, n), want)
+
+
+@pytest.mark.parametrize("M,N", [(1, 8), (63, 3), (65, 24), (4097, 1), (70000, 32), (300, 2056), (20000, 256), (129, 300)])
+def test_bias_gradient_against_float64(M, N):
+    rng = np.random.default_rng(M + N)
+    d = _bf(rng.standard_normal((M, N)))
+    db, g = U.Buf((M, N)).upload(d), U.Buf((N,), "f32").upload(np.ones(N))
+    ps.core.check(lib.ps_nn_bias_grad(db.p, M, N, g.p, None))
+    # FP32 partial sums: at most M roundings of values below the sum of magnitudes
+    assert np.abs(g.download() - 1.0 - d.astype(np.float64).sum(0)).max() <= 2.0 ** -24 * (np.abs(d).sum(0).max() * np.sqrt(M) + 8)
