@@ -12,7 +12,6 @@ from parallelstencil import unet as U
 from parallelstencil._lib import lib
 
 pytestmark = pytest.mark.gpu
-ps.ensure_device()
 
 
 def _bf(a):
