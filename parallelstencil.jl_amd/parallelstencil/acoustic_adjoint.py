@@ -153,15 +153,25 @@ class Acoustic2DInversion:
         self.snap = [(z(nx + 1, ny), z(nx, ny + 1)) for _ in range(self.seg)]
         # numbertype scalars
         self._t = np.float32 if core._numbertype_of(module) == core.Float32 else np.float64
+        self._plans = {}  # prepared launches by step and default stream
+
+    def _run(self, key, make):
+        """Runs the prepared launch `key` of the current default stream, made by make() on first use: a
+        step of this model takes a few microseconds, less than building its argument blocks anew."""
+        key = (key, core._stream_handle(None))
+        L = self._plans.get(key)
+        if L is None:
+            L = self._plans[key] = make()
+        L()
 
     # -------------------------------------------------------------- forward
     def _step(self, n, record=True):
         s, t = self.s, self._t
-        self.k_v(self.Vx, self.Vy, self.P, t(s.dt), t(s.rho), t(s.dx), t(s.dy), async_=True)
-        self.k_p(self.P, self.Vx, self.Vy, self.K, t(s.dt), t(s.dx), t(s.dy), async_=True)
-        self.k_inj(self.P, t(s.src[n]), s.isx, s.isy, ranges=((1, 1),), async_=True)
+        self._run("V", lambda: self.k_v.launcher(self.Vx, self.Vy, self.P, t(s.dt), t(s.rho), t(s.dx), t(s.dy)))
+        self._run("P", lambda: self.k_p.launcher(self.P, self.Vx, self.Vy, self.K, t(s.dt), t(s.dx), t(s.dy)))
+        self._run(("inject", n), lambda: self.k_inj.launcher(self.P, t(s.src[n]), s.isx, s.isy, ranges=((1, 1),)))
         if record:
-            self.k_rec(self.D, self.P, s.rx0, s.rdx, s.ry, n + 1, ranges=((1, s.nrec),), async_=True)
+            self._run(("record", n), lambda: self.k_rec.launcher(self.D, self.P, s.rx0, s.rdx, s.ry, n + 1, ranges=((1, s.nrec),)))
 
     def _reset_state(self):
         for A in (self.P, self.Vx, self.Vy):
@@ -207,11 +217,10 @@ class Acoustic2DInversion:
                 self.snap[n - n0][0].copy_(self.Vx, async_=True)
                 self.snap[n - n0][1].copy_(self.Vy, async_=True)
             for n in reversed(range(n0, n1)):
-                Vx1, Vy1 = self.snap[n - n0]
-                self.k_res(self.lP, self.D, self.Dobs, s.rx0, s.rdx, s.ry, n + 1, ranges=((1, s.nrec),), async_=True)
-                self.k_gk(self.gK, self.lP, Vx1, Vy1, t(s.dt), t(s.dx), t(s.dy), async_=True)
-                self.k_av(self.lVx, self.lVy, self.lP, self.K, t(s.dt), t(s.dx), t(s.dy), async_=True)
-                self.k_ap(self.lP, self.lVx, self.lVy, t(s.dt), t(s.rho), t(s.dx), t(s.dy), async_=True)
+                self._run(("residual", n), lambda: self.k_res.launcher(self.lP, self.D, self.Dobs, s.rx0, s.rdx, s.ry, n + 1, ranges=((1, s.nrec),)))
+                self._run(("K", n - n0), lambda: self.k_gk.launcher(self.gK, self.lP, *self.snap[n - n0], t(s.dt), t(s.dx), t(s.dy)))
+                self._run("lV", lambda: self.k_av.launcher(self.lVx, self.lVy, self.lP, self.K, t(s.dt), t(s.dx), t(s.dy)))
+                self._run("lP", lambda: self.k_ap.launcher(self.lP, self.lVx, self.lVy, t(s.dt), t(s.rho), t(s.dx), t(s.dy)))
         core.synchronize()
         return J, self.gK.to_host().astype(np.float64)
 
