@@ -56,3 +56,23 @@ def test_threads_transfer_at_once():
     for t in ts:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("shape,et", [((1,), ps.Float64), ((1001,), ps.Float32), ((33, 3), ps.Float64), ((1025, 70, 1), ps.Float32), ((130, 9, 7), ps.BFloat16),
+                                      ((65, 1, 9), ps.Bool), ((2, 70000), ps.Float64)])
+def test_device_copies(shape, et):
+    h = _host(shape, et, 4)
+    A, B = ps.zeros(*shape, eltype=et).copy_from(h), ps.zeros(*shape, eltype=et)
+    B.copy_(A)
+    assert np.array_equal(B.to_host(), h)
+
+
+@pytest.mark.parametrize("lo,hi", [((2, 1, 1), (33, 20, 9)), ((5, 3, 2), (30, 19, 8)), ((3, 4, 5), (3, 20, 5))])
+def test_device_copies_of_views(lo, hi):
+    # rows that start off a 16-byte boundary, and elements beside the view that must stay
+    ha, hb = _host((33, 20, 9), ps.Float64, 5), _host((40, 21, 9), ps.Float64, 6)
+    A, B = ps.zeros(33, 20, 9, eltype=ps.Float64).copy_from(ha), ps.zeros(40, 21, 9, eltype=ps.Float64).copy_from(hb)
+    box = tuple(slice(a - 1, b) for a, b in zip(lo, hi))
+    B.view(lo, hi).copy_(A.view(lo, hi))
+    hb[box] = ha[box]
+    assert np.array_equal(B.to_host(), hb) and np.array_equal(A.to_host(), ha)
