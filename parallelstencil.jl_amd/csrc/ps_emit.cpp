@@ -273,6 +273,11 @@ class Emitter {
   bool in_loop = false;  // inside the memopt stream loop
   // memopt register cache: key (arg, ox, oy, oz) -> register name
   std::map<std::tuple<int, int, int, int>, std::string> cache;
+  // arrays whose registers and tiles hold u/A for one uniform u instead of A (see quotient_arrays)
+  std::map<int, NodeP> quot_num;
+  bool load_cached = false;  // the last load() was served by the cache
+  void quotient_arrays(const std::vector<int>& arrays);
+  EV quotient(EV a, EV b);
   // scalar arguments used as uniform divisors: their reciprocal travels as a hidden argument
   std::map<int, Ty> rcp_params;
   bool fast_div = false;   // emitting the reciprocal form of a statement
@@ -471,6 +476,7 @@ std::string Emitter::offset(int ai, const std::vector<NodeP>& idx, std::string i
 }
 
 EV Emitter::load(const NodeP& n) {
+  load_cached = false;
   if (any_cell) {
     int cai;
     NodeP cidx;
@@ -541,7 +547,10 @@ EV Emitter::load(const NodeP& n) {
     }
     if (ok) {
       auto it = cache.find(std::make_tuple(ai, (int)off[0], (int)off[1], (int)off[2]));
-      if (it != cache.end()) return EV{it->second, value_ty(kinds[ai].dtype)};
+      if (it != cache.end()) {
+        load_cached = true;
+        return EV{it->second, value_ty(kinds[ai].dtype)};
+      }
     }
   }
   std::string ic[3];
@@ -654,10 +663,74 @@ bool rcp_safe32(float b) {
 
 // a / b. Uniform float divisors (scalar arguments the host accepted, literals) are divided
 // through their reciprocal (ps_divp) when the enclosing statement provides a fallback.
+// a / b for a divisor that is not uniform
+EV Emitter::quotient(EV a, EV b) {
+  if (a.t == Ty::Bool) a = cast(a, Ty::Int);
+  if (b.t == Ty::Bool) b = cast(b, Ty::Int);
+  Ty t = promote(a.t, b.t);
+  if (t == Ty::Int) t = Ty::F64;
+  if (K.opt.fastmath && (t == Ty::F64 || t == Ty::F32)) return EV{"(" + cast(a, t).c + " * ps_frcp(" + cast(b, t).c + "))", t};
+  return binary("/", a, b, nullptr);
+}
+
+// Read-only arrays that the kernel reads at several points, each time as the divisor of the same
+// scalar argument or literal (dt/Cp at the seven points of the reverse-mode diffusion step): the
+// memopt stream divides each value once, as it arrives, and keeps the quotient in its registers and
+// tiles. The quotients are the ones each use would have formed, so no bit changes; 7 divisions per
+// cell become one and the halo's share (reverse-mode diffusion3D at 256^3, gather kernel: GATHERUS).
+void Emitter::quotient_arrays(const std::vector<int>& arrays) {
+  quot_num.clear();
+  struct Use {
+    NodeP num;
+    std::string text;
+    std::set<std::string> points;
+    bool other = false;
+  };
+  std::map<int, Use> uses;
+  std::function<void(const NodeP&)> walk = [&](const NodeP& n) {
+    if (!n) return;
+    auto array_of = [&](const NodeP& x) { return x && x->k == NK::Index && x->a[0]->k == NK::Ident ? field_index(x->a[0]->s) : -1; };
+    if (n->k == NK::Binary && n->s == "/") {
+      const int ai = array_of(n->a[1]);
+      const NodeP& u = n->a[0];
+      if (ai >= 0) {
+        Use& s = uses[ai];
+        bool uniform = u->k == NK::Num;
+        if (u->k == NK::Ident) {
+          auto it = K.param_index.find(u->s);
+          uniform = it != K.param_index.end() && !kinds[it->second].is_field;
+        }
+        const std::string text = to_julia(u);
+        if (!uniform || (s.num && text != s.text)) s.other = true;
+        s.num = u;
+        s.text = text;
+        s.points.insert(to_julia(n->a[1]));
+        walk(u);
+        for (size_t i = 1; i < n->a[1]->a.size(); ++i) walk(n->a[1]->a[i]);
+        return;
+      }
+    }
+    const int ai = array_of(n);
+    if (ai >= 0) uses[ai].other = true;
+    for (auto& c : n->a) walk(c);
+  };
+  walk(K.body);
+  for (int ai : arrays) {
+    auto it = uses.find(ai);
+    if (it == uses.end() || it->second.other || it->second.points.size() < 2) continue;
+    const Ty at = value_ty(kinds[ai].dtype);
+    if (!is_float(at) || locals.count(it->second.text)) continue;
+    const Ty nt = expr(it->second.num).t;
+    if (promote(nt == Ty::Bool ? Ty::Int : nt, at) != at) continue;  // the quotient is of the array's own type
+    quot_num[ai] = it->second.num;
+  }
+}
+
 EV Emitter::divide(const NodeP& n) {
   EV a = expr(n->a[0]);
   const NodeP& d = n->a[1];
   EV b = expr(d);
+  if (in_loop && load_cached && d->k == NK::Index && d->a[0]->k == NK::Ident && quot_num.count(field_index(d->a[0]->s))) return b;
   if (a.t == Ty::Bool) a = cast(a, Ty::Int);
   if (b.t == Ty::Bool) b = cast(b, Ty::Int);
   Ty t = promote(a.t, b.t);
@@ -678,7 +751,7 @@ EV Emitter::divide(const NodeP& n) {
       double r = t == Ty::F32 ? (double)(1.0f / (float)v) : 1.0 / v;
       return EV{"(" + cast(a, t).c + " * " + hexlit(r, t) + ")", t};
     }
-    return EV{"(" + cast(a, t).c + " * ps_frcp(" + cast(b, t).c + "))", t};
+    return quotient(a, b);
   }
   if (fast_div && d->k == NK::Ident && !locals.count(d->s)) {
     auto it = K.param_index.find(d->s);
@@ -2025,6 +2098,15 @@ void Emitter::emit_memopt_body(int L) {
   if (!V.checked)
     for (auto& kv : mm.ro_offsets) collect(kv.first, kv.second, false);
 
+  std::vector<int> streamed;
+  for (auto& P : pts) streamed.push_back(P.ai);
+  if (!V.checked) quotient_arrays(streamed);
+  // the value of array ai that registers and tiles hold for the loaded value x
+  auto held = [&](int ai, const std::string& x) {
+    auto it = quot_num.find(ai);
+    return it == quot_num.end() ? x : quotient(expr(it->second), EV{x, value_ty(kinds[ai].dtype)}).c;
+  };
+
   // LDS tiles: planes of optvars read at several (ox, oy) columns are staged in LDS once per
   // step; each thread contributes its register value ("own" column), the halo runs are loaded
   // by the first lanes of the block.
@@ -2220,7 +2302,7 @@ void Emitter::emit_memopt_body(int L) {
   for (auto& c : cols) {
     int w = c.zhi - c.zlo + 1;
     for (int k = 0; k + 1 < w; ++k)
-      o << pad() << c.name << "_" << k << " = " << ldq(c, "ps_zb + (" + std::to_string(c.zlo + k) + ")", "") << ";\n";
+      o << pad() << c.name << "_" << k << " = " << held(c.ai, ldq(c, "ps_zb + (" + std::to_string(c.zlo + k) + ")", "")) << ";\n";
     for (int d = 0; d < PD; ++d)
       o << pad() << c.name << "_n" << d << " = " << ldq(c, "ps_zb + (" + std::to_string(c.zhi + d) + ")", within(d)) << ";\n";
   }
@@ -2267,6 +2349,62 @@ void Emitter::emit_memopt_body(int L) {
     if (kinds[t.ai].dtype == PS_BF16) v = "ps_bf16_ld(" + v + ")";
     return v;
   };
+  // A body of several guarded statements (the gather form of a derivative: one per stencil neighbour) also
+  // comes without the guards, for the steps of wavefronts in which every guard holds for every cell: the
+  // loads of all statements are then issued together instead of one by one behind their branches. The
+  // guards' conditions are split into those on the streamed index, uniform in a step, and those on the
+  // others, evaluated once before the stream.
+  NodeP unguarded;
+  std::vector<std::string> gz;
+  if (!V.checked && !pass1) {
+    std::set<std::string> gxy, gzs;
+    int guards = 0;
+    bool ok = true;
+    std::function<bool(const NodeP&, bool&, bool&)> pure = [&](const NodeP& n, bool& z, bool& xy) -> bool {
+      if (n->k == NK::Ident) {
+        if (n->s == kIdx[L]) z = true;
+        else if (n->s == kIdx[0] || n->s == kIdx[1] || n->s == kIdx[2]) xy = true;
+        return !locals.count(n->s) && field_index(n->s) < 0;
+      }
+      if (n->k == NK::Call) return n->s == "size";
+      if (n->k != NK::Num && n->k != NK::Cmp && n->k != NK::Binary && n->k != NK::Unary) return false;
+      for (auto& c : n->a)
+        if (!pure(c, z, xy)) return false;
+      return true;
+    };
+    std::function<void(const NodeP&)> conds = [&](const NodeP& c) {
+      if (c->k == NK::And) {
+        for (auto& x : c->a) conds(x);
+        return;
+      }
+      bool z = false, xy = false;
+      if (c->k != NK::Cmp || !pure(c, z, xy) || (z && xy)) {
+        ok = false;
+        return;
+      }
+      (z ? gzs : gxy).insert(expr(c).c);
+    };
+    std::function<void(const NodeP&, const NodeP&)> strip = [&](const NodeP& b, const NodeP& out) {
+      for (auto& st : b->a) {
+        if (st->k == NK::If && !(st->a.size() > 2 && st->a[2])) {
+          ++guards;
+          conds(st->a[0]);
+          strip(st->a[1], out);
+        } else {
+          out->a.push_back(st);
+        }
+      }
+    };
+    NodeP out = mk(NK::Block);
+    strip(K.body, out);
+    if (ok && guards >= 2) {
+      unguarded = out;
+      gz.assign(gzs.begin(), gzs.end());
+      o << pad() << "const bool ps_gxy = __all(" << (V.lds ? "!ps_act || (" : "(") << "true";
+      for (auto& g : gxy) o << " && " << g;
+      o << "));\n";
+    }
+  }
   auto emit_loop = [&](const std::string& to, bool fast) {
     o << pad() << "for (; " << lc << " < " << to << "; ++" << lc << ") {\n";
     ++ind;
@@ -2274,7 +2412,7 @@ void Emitter::emit_memopt_body(int L) {
     if (!fast) o << pad() << "const bool ps_more = " << lc << " + " << PD << " < ps_ze;\n";
     for (auto& c : cols) {
       int w = c.zhi - c.zlo + 1;
-      o << pad() << c.name << "_" << (w - 1) << " = " << c.name << "_n0;\n";
+      o << pad() << c.name << "_" << (w - 1) << " = " << held(c.ai, c.name + "_n0") << ";\n";
       for (int d = 0; d + 1 < PD; ++d) o << pad() << c.name << "_n" << d << " = " << c.name << "_n" << d + 1 << ";\n";
       const std::string z = lc + " + (" + std::to_string(c.zhi + PD) + ")";
       o << pad() << c.name << "_n" << PD - 1 << " = " << (fast ? ldq_fast(c, z) : ldq(c, z, "ps_more && ")) << ";\n";
@@ -2287,7 +2425,7 @@ void Emitter::emit_memopt_body(int L) {
           << "] = " << c.name << "_" << (t.oz - c.zlo) << ";\n";
         for (int j = 0; j < t.nslots; ++j) {
           std::string S = t.name + "_s" + std::to_string(j);
-          o << pad() << "if (" << S << "_v) " << t.name << "[ps_buf][" << S << "_l] = " << S << "_h0;\n";
+          o << pad() << "if (" << S << "_v) " << t.name << "[ps_buf][" << S << "_l] = " << held(t.ai, S + "_h0") << ";\n";
           for (int d = 0; d + 1 < PD; ++d) o << pad() << S << "_h" << d << " = " << S << "_h" << d + 1 << ";\n";
           const std::string z = lc + " + (" + std::to_string(t.oz + PD) + ")";
           // lanes without a halo slot skip the load (whole waves of them branch around it)
@@ -2324,7 +2462,21 @@ void Emitter::emit_memopt_body(int L) {
       o << pad() << "if (ps_act) {\n";
       ++ind;
     }
+    if (unguarded) {
+      o << pad() << "if (ps_gxy";
+      for (auto& g : gz) o << " && " << g;
+      o << ") {\n";
+      ++ind;
+      block(unguarded);
+      --ind;
+      o << pad() << "} else {\n";
+      ++ind;
+    }
     block(K.body);
+    if (unguarded) {
+      --ind;
+      o << pad() << "}\n";
+    }
     if (V.lds) {
       --ind;
       o << pad() << "}\n";
