@@ -147,3 +147,38 @@ def test_bias_gradient_against_float64(M, N):
     ps.core.check(lib.ps_nn_bias_grad(db.p, M, N, g.p, None))
     # FP32 partial sums: at most M roundings of values below the sum of magnitudes
     assert np.abs(g.download() - 1.0 - d.astype(np.float64).sum(0)).max() <= 2.0 ** -24 * (np.abs(d).sum(0).max() * np.sqrt(M) + 8)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 8), (257, 3, 32), (1000, 4, 24), (70001, 2, 512), (5, 3, 40)])
+def test_thin_results_against_float64(M, N, K):
+    # K FP32 products and sums of BF16 values, rounded once to BF16 (2^-8 of the value) at the end
+    rng = np.random.default_rng(M + N + K)
+    a, w, bias = _bf(rng.standard_normal((M, K))), _bf(rng.standard_normal((K, N))), rng.standard_normal(N).astype(np.float32)
+    A, Wb, bb = U.Buf((M, K)).upload(a), U.Buf((K, N)).upload(w), U.Buf((N,), "f32").upload(bias)
+    ref = a.astype(np.float64) @ w.astype(np.float64)
+    mag = np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64) + 4
+    for epi, want in ((U.EPI_BF16, ref), (U.EPI_BIAS, ref + bias), (U.EPI_BIAS_RELU, np.maximum(ref + bias, 0))):
+        C = U.Buf((M, N))
+        U.gemm(M, N, K, A, K, 1, Wb, N, 1, C, N, bb, epi)
+        assert (np.abs(C.download() - want) <= 2.0 ** -8 * np.abs(want) + 2.0 ** -22 * mag).all(), epi
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 1), (300, 32, 3), (70001, 24, 4), (65, 512, 2)])
+def test_thin_sums_against_float64(M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    a, w = _bf(rng.standard_normal((M, K))), _bf(rng.standard_normal((N, K)))
+    A, Wb, C = U.Buf((M, K)).upload(a), U.Buf((N, K)).upload(w), U.Buf((M, N))
+    U.gemm(M, N, K, A, K, 1, Wb, 1, K, C, N)
+    ref = a.astype(np.float64) @ w.T.astype(np.float64)
+    assert (np.abs(C.download() - ref) <= 2.0 ** -8 * np.abs(ref) + 2.0 ** -20).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 1, 300), (32, 3, 131072), (24, 4, 1000), (2048, 2, 700), (2056, 2, 700)])
+def test_thin_gradients_against_float64(M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    a, d = _bf(rng.standard_normal((K, M))), _bf(rng.standard_normal((K, N)))
+    A, D, G = U.Buf((K, M)).upload(a), U.Buf((K, N)).upload(d), U.Buf((M, N), "f32").upload(np.ones((M, N)))
+    U.gemm(M, N, K, A, 1, M, D, N, 1, G, N, epi=U.EPI_F32_ADD, splitk=3)
+    ref = a.astype(np.float64).T @ d.astype(np.float64)
+    # FP32 sums of K products in any order, as for the weight gradient above
+    assert np.abs(G.download() - 1.0 - ref).max() <= 8 * 2.0 ** -24 * (K + 4 * np.sqrt(K))
