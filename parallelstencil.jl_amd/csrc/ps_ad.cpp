@@ -846,6 +846,87 @@ class Ad {
       });
     }
   }
+  // e with the uniform factors of its terms gathered: a sum of products of loads, each times one
+  // expression of scalar arguments and literals (which the host evaluates once per launch), terms with
+  // the same loads merged. The chain rule leaves (((-((g*(dt/Cp))/dx))/dx)*(-lam)) and sums of six of
+  // them at a cell; gathered they are one load product times one number. The quantity is the same up to
+  // the rounding of the factors, whose order is this transformation's own. An expression with a
+  // comparison among its factors (Bool * x is a strong zero) is left as it is.
+  bool uniform(const NodeP& n) const {
+    if (n->k == NK::Num) return true;
+    if (n->k == NK::Ident) {
+      auto it = K.param_index.find(n->s);
+      return it != K.param_index.end() && !K.accessed.count(n->s) && !locals.count(n->s) && K.def.params[it->second].annot.find("Bool") == std::string::npos;
+    }
+    if (n->k == NK::Unary && (n->s == "-" || n->s == "+")) return uniform(n->a[0]);
+    if (n->k == NK::Binary && (n->s == "+" || n->s == "-" || n->s == "*" || n->s == "/")) return uniform(n->a[0]) && uniform(n->a[1]);
+    return false;
+  }
+  struct Term {
+    std::vector<NodeP> f;  // factors that vary from cell to cell
+    NodeP u;               // uniform factor, null for 1
+    bool minus = false;
+  };
+  static NodeP one_times(const NodeP& u) { return mk(NK::Binary, "*", {fnum(1.0), u}); }  // a float even where u is an integer
+  bool factors(const NodeP& n, Term& t) const {
+    if (uniform(n)) {
+      t.u = t.u ? mk(NK::Binary, "*", {t.u, clone(n)}) : one_times(clone(n));
+      return true;
+    }
+    if (n->k == NK::Binary && n->s == "*") return factors(n->a[0], t) && factors(n->a[1], t);
+    if (n->k == NK::Binary && n->s == "/" && uniform(n->a[1])) {
+      if (!factors(n->a[0], t)) return false;
+      t.u = mk(NK::Binary, "/", {t.u ? t.u : fnum(1.0), clone(n->a[1])});
+      return true;
+    }
+    if (n->k == NK::Unary && n->s == "-") {
+      t.minus = !t.minus;
+      return factors(n->a[0], t);
+    }
+    if (n->k == NK::Cmp || n->k == NK::And || n->k == NK::Or || (n->k == NK::Unary && n->s == "!")) return false;
+    t.f.push_back(n);
+    return true;
+  }
+  bool terms(const NodeP& n, bool minus, std::vector<Term>& out) const {
+    if (n->k == NK::Binary && (n->s == "+" || n->s == "-") && !uniform(n))
+      return terms(n->a[0], minus, out) && terms(n->a[1], n->s == "-" ? !minus : minus, out);
+    if (n->k == NK::Unary && n->s == "-" && !uniform(n)) return terms(n->a[0], !minus, out);
+    Term t;
+    if (!factors(n, t)) return false;
+    if (minus) t.minus = !t.minus;
+    out.push_back(t);
+    return true;
+  }
+  NodeP gathered(const NodeP& e) const {
+    std::vector<Term> ts;
+    if (!terms(e, false, ts)) return e;
+    std::vector<std::string> order;
+    std::map<std::string, std::vector<Term>> groups;
+    for (auto& t : ts) {
+      std::string key;
+      for (auto& f : t.f) key += to_julia(f) + ";";
+      if (!groups.count(key)) order.push_back(key);
+      groups[key].push_back(t);
+    }
+    NodeP sum;
+    for (auto& key : order) {
+      auto& g = groups[key];
+      NodeP prod, u;
+      for (auto& f : g[0].f) prod = prod ? mk(NK::Binary, "*", {prod, clone(f)}) : clone(f);
+      const bool minus = g[0].minus;  // of the group: the others' signs count against it
+      if (g.size() == 1) {
+        u = g[0].u;
+      } else {
+        for (auto& t : g) {
+          NodeP x = t.u ? t.u : fnum(1.0);
+          u = !u ? x : mk(NK::Binary, t.minus == minus ? "+" : "-", {u, x});
+        }
+      }
+      NodeP x = prod && u ? mk(NK::Binary, "*", {prod, u}) : prod ? prod : u ? u : fnum(1.0);
+      sum = !sum ? (minus ? neg(x) : x) : mk(NK::Binary, minus ? "-" : "+", {sum, x});
+    }
+    return sum ? sum : e;
+  }
   // Copy of e at the point i = j - o: parallel index d becomes (index - o_d).
   NodeP shift(const NodeP& e, const long long o[3]) const {
     std::function<NodeP(const NodeP&)> f = [&](const NodeP& n) -> NodeP {
@@ -886,7 +967,7 @@ class Ad {
             cond = conj(cond, cmp(i, "<", mk(NK::Binary, "+", {ident(r0), ident(rl)})));
           }
           if (w.cond) cond = conj(cond, shift(w.cond, o));
-          auto then = mk(NK::Block, "", {assign(ident(acc), add(ident(acc), shift(p.value(), o)))});
+          auto then = mk(NK::Block, "", {assign(ident(acc), add(ident(acc), shift(gathered(p.value()), o)))});
           body->a.push_back(mk(NK::If, "", {cond, then, nullptr}));
         }
         pending.clear();

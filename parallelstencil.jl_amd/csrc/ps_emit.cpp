@@ -2097,6 +2097,10 @@ void Emitter::emit_memopt_body(int L) {
   // variant keeps their plain (checked) loads
   if (!V.checked)
     for (auto& kv : mm.ro_offsets) collect(kv.first, kv.second, false);
+  // and so are the elements that the thread alone updates in place: their load would otherwise wait for
+  // memory between the step's barrier and its store (reverse-mode diffusion3D at 256^3: 172 us, OWNUS)
+  if (!V.checked && V.noalias)
+    for (auto& kv : mm.own_offsets) collect(kv.first, kv.second, false);
 
   std::vector<int> streamed;
   for (auto& P : pts) streamed.push_back(P.ai);

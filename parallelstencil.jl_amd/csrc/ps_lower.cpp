@@ -738,6 +738,31 @@ static void memopt_analysis(Kernel& K) {
       ++it;
     }
   }
+  bool loops = false;
+  walk(K.body, [&](const NodeP& x) { loops = loops || x->k == NK::For || (x->k == NK::Macro && x->s == "ps_atomic_add"); });
+  for (auto& A : K.written) {
+    if (loops || !K.param_index.count(A)) continue;
+    std::vector<NodeP> sets;  // the assignments to A
+    int all = 0, inside = 0;
+    auto is_A = [&](const NodeP& x) { return x->k == NK::Index && x->a[0]->k == NK::Ident && x->a[0]->s == A; };
+    walk(K.body, [&](const NodeP& x) {
+      if (x->k == NK::Assign && is_A(x->a[0])) sets.push_back(x);
+      if (is_A(x)) ++all;
+    });
+    if (sets.size() != 1 || !sets[0]->s.empty()) continue;
+    const NodeP& target = sets[0]->a[0];
+    const std::string text = to_julia(target);
+    walk(sets[0]->a[1], [&](const NodeP& x) { inside += is_A(x) && to_julia(x) == text; });
+    if (inside == 0 || inside + 1 != all) continue;
+    int off[3] = {0, 0, 0};
+    bool own = (int)target->a.size() - 1 >= nd;
+    for (int d = 0; own && d + 1 < (int)target->a.size(); ++d) {
+      Aff a = affine(target->a[1 + d]);
+      own = d < nd ? a.ok && a.var == d : a.ok && a.var < 0 && a.c == 1;
+      if (d < nd) off[d] = (int)a.c;
+    }
+    if (own) mm.own_offsets[A][nd == 3 ? std::make_pair(off[0], off[1]) : std::make_pair(off[0], 0)][off[nd - 1]] += 1;
+  }
   for (auto& A : mm.optvars) {
     std::vector<std::pair<int, int>> sr(3, {0, 0});
     bool first = true;

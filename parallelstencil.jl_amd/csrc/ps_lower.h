@@ -38,6 +38,9 @@ struct MemoptMeta {
   std::map<std::string, std::map<std::pair<int, int>, std::map<int, int>>> offsets;
   // same for the read-only arrays that are not optvars (register prefetch only)
   std::map<std::string, std::map<std::pair<int, int>, std::map<int, int>>> ro_offsets;
+  // written arrays that one assignment updates in place (A[p] = ... A[p] ..., read nowhere else), at p's
+  // offset, in the same form: no other thread writes the element, so it can be read ahead too
+  std::map<std::string, std::map<std::pair<int, int>, std::map<int, int>>> own_offsets;
   std::vector<std::string> shmem_optvars;
   std::map<std::string, bool> use_shmemhalos;
 };
