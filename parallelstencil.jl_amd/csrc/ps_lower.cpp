@@ -291,7 +291,7 @@ static void read_options(Options& o, const JVal& j) {
     else if (k == "inbounds") o.inbounds = v.b;
     else if (k == "padding") o.padding = v.b;
     else if (k == "memopt") o.memopt = v.b;
-    else if (k == "loopsize") o.loopsize = (int)v.n;
+    else if (k == "loopsize") o.loopsize = (int)v.n, o.loopsize_given = true;
     else if (k == "loopdim") o.loopdim = (int)v.n;
     else if (k == "optvars") {
       o.optvars.clear();
@@ -364,7 +364,7 @@ static void apply_prefix_kwargs(Options& o, const KernelDef& kd) {
     else if (k == "inbounds") o.inbounds = as_bool();
     else if (k == "padding") o.padding = as_bool();
     else if (k == "ndims") o.ndims = as_int();
-    else if (k == "loopsize") o.loopsize = as_int();
+    else if (k == "loopsize") o.loopsize = as_int(), o.loopsize_given = true;
     else if (k == "loopdim") o.loopdim = as_int();
     else if (k == "optvars") {
       o.optvars.clear();
@@ -1437,7 +1437,7 @@ std::string Variant::key() const {
   char b[96];
   std::snprintf(b, sizeof b, "m%dc%di%da%dt%dl%d_%dx%dn%do%du%dg%dz%d", memopt, checked, idx64, noalias, maxthreads, lds, bx, by, nt, off32, u24, cx,
                 cz);
-  return std::string(b) + "d" + divmode + (padbits.empty() ? "" : "p" + padbits) + (sclass.empty() ? "" : "s" + sclass);
+  return std::string(b) + (loopsize ? "k" + std::to_string(loopsize) : "") + "d" + divmode + (padbits.empty() ? "" : "p" + padbits) + (sclass.empty() ? "" : "s" + sclass);
 }
 
 }  // namespace ps

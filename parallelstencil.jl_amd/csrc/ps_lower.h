@@ -54,6 +54,7 @@ struct Options {
   bool padding = false;
   bool memopt = false;
   int loopsize = 32;
+  bool loopsize_given = false;            // a given loopsize is the one launched
   int loopdim = 0;
   std::vector<std::string> optvars;
   std::map<std::string, std::vector<std::pair<int, int>>> optranges;
@@ -129,6 +130,7 @@ struct Variant {
   int maxthreads = 256;   // __launch_bounds__
   bool lds = false;       // memopt: stage x-y neighbours of optvars through LDS tiles
   bool nt = false;        // nontemporal stores for array writes
+  int loopsize = 0;       // memopt: planes streamed by a thread (0: the kernel's loopsize)
   // plain kernels: affine accesses address an SGPR base (array + uniform offset) plus a 32-bit
   // per-thread byte offset; the host sets it when every thread's cell offset is non-negative and
   // every byte offset of the launch box fits in 31 bits

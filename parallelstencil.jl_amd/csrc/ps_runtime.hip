@@ -1545,11 +1545,34 @@ Plan plan_launch(const Kernel& K, const ps_arg* args, int nargs, const ps_launch
     P.lthreads[d] = P.nthreads[d];
     P.lblocks[d] = P.nblocks[d];
   }
+  // memopt launches whose grid leaves CUs idle stream fewer planes per thread than the kernel's
+  // (default) loopsize: 16 or 8 while fewer than 2M threads run (four times what the GPU holds),
+  // 4 and 2 where even 8 planes leave less than half of it. geometry() keeps reporting the loopsize's.
+  // us with 2 / 4 / 8 / 16 / 32 planes, diffusion3D FP64: 32^3 4.0 / 4.9 / 7.6 / 13.5 / 21.3, 64^3 3.9 / 5.1 / 7.7 / 12.8 /
+  // 23.3, 128^3 14.2 / 13.0 / 13.7 / 16.9 / 27.5, 512 x 100 x 40 15.1 / 12.9 / 13.2 / 20.6 / 37.3, 256^3 95 / 84.5 / 83.0 /
+  // 83.5 / 88.8 (its reverse mode 141 / 126 / 123 / 120 / 142), 512^3 768 / 666 / 612 / 614 / 602.
+  int stream = 0;
+  if (memopt && !user_geom && !K.opt.loopsize_given && P.nthreads[K.mm.loopdim - 1] == 1) {
+    const int Ld = K.mm.loopdim - 1;
+    int64_t plane = 1;
+    for (int d = 0; d < 3; ++d)
+      if (d != Ld) plane *= (int64_t)P.nthreads[d] * P.nblocks[d];
+    auto threads = [&](int ls) { return plane * ((len[Ld] + ls - 1) / ls); };
+    int ls = K.mm.loopsize;
+    while (ls > 8 && threads(ls) < (2 << 20)) ls /= 2;
+    if (ls == 8 && threads(8) < (1 << 18)) ls = threads(4) < (1 << 17) ? 2 : 4;
+    const int64_t chunks = (len[Ld] + ls - 1) / ls;
+    if (ls != K.mm.loopsize && chunks <= 65535) {
+      stream = ls;
+      P.lblocks[Ld] = (int32_t)chunks;
+    }
+  }
   if ((int64_t)P.nthreads[0] * P.nthreads[1] * P.nthreads[2] > 1024) throw PsError(PS_EARGUMENT, "at most 1024 threads per block are supported");
   if (P.nblocks[1] > 65535 || P.nblocks[2] > 65535) throw PsError(PS_EARGUMENT, "nblocks in y and z must not exceed 65535");
   // variant
   Variant v;
   v.memopt = memopt;
+  v.loopsize = stream;
   if (memopt && K.opt.lds && !K.mm.shmem_optvars.empty() && K.mm.loopdim == 3 && P.nthreads[2] == 1) {
     v.lds = true;
     v.bx = P.nthreads[0];

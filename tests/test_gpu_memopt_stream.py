@@ -1,0 +1,95 @@
+"""memopt streams against plain kernels, bit for bit, over the grids where the number of planes per
+thread changes (2, 4, 8, 16 and 32, and remainders of each), for a stencil and for in-place updates read
+ahead; quotients of one scalar by an array taken once per value; the gather form of a derivative with
+its streams against the atomic scatter form."""
+import numpy as np
+import pytest
+
+import parallelstencil as ps
+from parallelstencil import workloads as W
+
+pytestmark = pytest.mark.gpu
+MOD = __name__
+ps.init_parallel_stencil(ps.AMDGPU, ps.Float64, 3, module=MOD)
+DIMS = [(20, 17, 9), (32, 32, 32), (64, 64, 33), (96, 96, 45), (128, 128, 70), (127, 95, 63), (300, 20, 37), (200, 130, 61), (256, 200, 99)]
+
+
+def _rand(dims, seed, lo=0.0):
+    return ps.zeros(*dims, eltype=ps.Float64).copy_from(lo + np.random.default_rng(seed).random(dims))
+
+
+@pytest.mark.parametrize("dims", DIMS)
+def test_stencil_matches_plain(dims):
+    T, Cp = _rand(dims, 1), _rand(dims, 2, 1.0)
+    outs = []
+    for memopt in (False, True):
+        T2 = _rand(dims, 3)
+        W.define_diffusion3d(memopt, MOD)(T2, T, Cp, 1.1, 0.01, 0.1, 0.2, 0.3)
+        outs.append(T2.to_host())
+    assert np.array_equal(*outs)
+
+
+@pytest.mark.parametrize("dims", DIMS)
+def test_in_place_updates_match_plain(dims):
+    nx, ny, nz = dims
+    outs = []
+    for memopt in (False, True):
+        P, Vx, Vy, Vz = (_rand(d, i) for i, d in enumerate((dims, (nx + 1, ny, nz), (nx, ny + 1, nz), (nx, ny, nz + 1))))
+        kV, kP = W.define_acoustic3d(MOD, memopt)
+        for _ in range(3):
+            kV(Vx, Vy, Vz, P, 0.01, 1.3, 0.1, 0.2, 0.3)
+            kP(P, Vx, Vy, Vz, 0.01, 0.9, 0.1, 0.2, 0.3)
+        outs.append([A.to_host() for A in (P, Vx, Vy, Vz)])
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+
+
+QUOT = """
+@parallel_indices (ix,iy,iz) function quotients!(B, A, C, s)
+    if (1 < ix < size(A,1) && 1 < iy < size(A,2) && 1 < iz < size(A,3))
+        B[ix,iy,iz] = B[ix,iy,iz] + A[ix-1,iy,iz]*(s/C[ix-1,iy,iz]) + A[ix+1,iy,iz]*(s/C[ix+1,iy,iz]) + A[ix,iy-1,iz]*(s/C[ix,iy-1,iz]) - A[ix,iy,iz-1]*(s/C[ix,iy,iz-1]) + s/C[ix,iy,iz+1]
+    end
+    return
+end
+"""
+
+
+@pytest.mark.parametrize("fastmath", [False, True])
+@pytest.mark.parametrize("dims", [(20, 17, 9), (128, 40, 70), (256, 64, 33)])
+def test_quotients_by_an_array_match_plain(dims, fastmath):
+    A, C = _rand(dims, 1), _rand(dims, 2, -0.5)  # divisors of both signs, some near zero
+    h = C.to_host()
+    h[3, 4, 5], h[4, 4, 5] = 0.0, np.inf
+    C.copy_from(h)
+    outs = []
+    for memopt in (False, True):
+        B = _rand(dims, 3)
+        ps.core._define("parallel_indices", QUOT, {"memopt": memopt, "fastmath": fastmath}, MOD)(B, A, C, 0.7)
+        outs.append(B.to_host())
+    if fastmath:
+        # contraction may differ between the two kernels: each of the six terms (large where C is near
+        # zero, and they cancel) within a few roundings, so 16 eps of the sum of their magnitudes
+        a, q = A.to_host(), 0.7 / np.abs(np.where(h == 0, np.nan, h))
+        mag = 2.0 + sum(np.roll(q * a, s, ax) for s, ax in ((1, 0), (-1, 0), (1, 1), (1, 2))) + np.roll(q, -1, 2)
+        ok = np.isfinite(outs[0]) & np.isfinite(mag)
+        assert np.array_equal(np.isfinite(outs[0]), np.isfinite(outs[1]))
+        assert (np.abs(outs[0] - outs[1])[ok] <= 16 * 2.0 ** -52 * mag[ok]).all()
+    else:
+        assert np.array_equal(*outs, equal_nan=True)
+
+
+@pytest.mark.parametrize("memopt", [False, True])
+@pytest.mark.parametrize("dims", DIMS[:7])
+def test_gather_matches_scatter(dims, memopt):
+    k = W.define_diffusion3d(memopt, MOD)
+    d = k._derivative("Reverse", {"T2": "DuplicatedNoNeed", "T": "DuplicatedNoNeed"})
+    T, T2, Cp = _rand(dims, 1), _rand(dims, 2), _rand(dims, 3, 1.0)
+    outs = []
+    for gather in (False, True):
+        S, R = _rand(dims, 4, -0.5), _rand(dims, 5)
+        d.use_gather = gather
+        d(T2, T, Cp, 1.1, 0.01, 0.1, 0.2, 0.3, S, R)
+        outs.append((S.to_host(), R.to_host()))
+    assert np.array_equal(outs[0][0], outs[1][0])
+    # seven products a cell, each a few roundings, in either order: 1e-14 of the largest term (about 5)
+    assert np.abs(outs[0][1] - outs[1][1]).max() <= 1e-13
