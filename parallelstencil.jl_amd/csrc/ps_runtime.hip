@@ -1674,7 +1674,7 @@ Plan plan_launch(const Kernel& K, const ps_arg* args, int nargs, const ps_launch
     // x groups (Variant::cx): with automatic geometry and a body of array assignments under
     // x-interval masks, each thread takes cx adjacent x cells (by default 4 when the narrowest
     // array has 2- or 4-byte elements: 8 or 16 bytes per thread, whose accesses merge into wide
-    // loads; FP64 arrays keep one cell, where groups measured slower)
+    // loads; FP64 arrays take z cells)
     bool cell = false;
     int64_t es = 8;
     for (int i = 0; i < nargs; ++i)
@@ -1683,16 +1683,24 @@ Plan plan_launch(const Kernel& K, const ps_arg* args, int nargs, const ps_launch
         es = std::min<int64_t>(es, elsize(args[i].field.dtype));
       }
     if (ok && !user_geom && !cell && groupable_body(K)) {
-      // Cells per thread. FP32 and BFloat16: 4 x cells. FP64 (3-D groups, rows of at least 256
-      // cells): z cells, twice the stencil's z reach (a thread then reads 1.5 planes per cell) and
-      // at most 8, so that a z plane that several of the thread's cells read is one load; and 2 x
-      // cells with them when the stencil reaches 2 cells along x. Measured at the sustained clock:
+      // Cells per thread. FP32 and BFloat16: 4 x cells. FP64 (3-D groups): z cells, twice the
+      // stencil's z reach (a thread then reads 1.5 planes per cell) and at most 8, so that a z plane
+      // that several of the thread's cells read is one load; and 2 x cells with them when the stencil
+      // reaches 2 cells along x. Measured at the sustained clock:
       // diffusion3D 512^3 (reaches 2 and 2) 0.860 ms per step with one cell, 0.739 / 0.684 /
       // 0.704 with 2 / 4 / 8 z cells, 0.652 with 2 x 4; acoustic3D 384^3 (reaches 1 and 1)
       // 1.026, 0.961 with 2 z cells, 0.998 with 4, 1.001 with 2 x 2. FP32 and BFloat16 groups
       // were 10-15% slower with z cells, and Stokes3D at 127^3 (rows of 127 cells: the edge block
       // column and the threads before the first interior group double the waves) 4% slower.
-      const bool fp64 = es >= 8 && len[0] >= 256 && groupable_body(K, true);
+      // FP64 rows of 160 to 255 cells take z cells from 4e6 cells on, where the launch still has waves
+      // enough with a quarter of them (us, one cell / z cells: diffusion3D 253x190x127 30.4 / 28.6,
+      // 192^3 36.1 / 32.6, 255^3 107 / 87, 255x512x512 442 / 333; acoustic3D compute_V 160^3 46 / 41,
+      // 192^3 86 / 67, 255x320x320 326 / 259, compute_P 0 to 10% faster). Shorter rows lose as often as
+      // they gain: 100x255x255 compute_V 65 / 72, diffusion3D 49 / 37; 63x255x255 33 / 42 and 25 / 31.
+      // 2 x cells pay from 12e6 cells on: 300x200x128 37.6 us with 1 x 4 and 40.6 with 2 x 4,
+      // 512x100x40 12.1 and 12.7, 192x255x255 72.7 and 72.4, 255x512x512 349 and 333.
+      const int64_t cells = len[0] * len[1] * len[2];
+      const bool fp64 = es >= 8 && (len[0] >= 256 || (len[0] >= 160 && cells >= 4000000)) && groupable_body(K, true);
       int cz = 1;
       if (K.opt.cells_z != 0) cz = K.opt.cells_z;
       else if (fp64) {
@@ -1700,7 +1708,7 @@ Plan plan_launch(const Kernel& K, const ps_arg* args, int nargs, const ps_launch
         cz = reach == 0 ? 1 : reach == 1 ? 2 : reach == 2 ? 4 : 8;
       }
       int cx = K.opt.cells_x;
-      if (cx == 0) cx = es < 8 ? 4 : fp64 && cz > 1 && idx_span(K, 0) >= 2 ? 2 : 1;
+      if (cx == 0) cx = es < 8 ? 4 : fp64 && cz > 1 && cells >= 12000000 && idx_span(K, 0) >= 2 ? 2 : 1;
       if (len[0] < 2 * (int64_t)cx) cx = 1;
       if (cz > 1 && (P.nthreads[2] != 1 || len[2] < 2 * (int64_t)cz || !groupable_body(K, true))) cz = 1;
       if (cx > 1 || cz > 1) {

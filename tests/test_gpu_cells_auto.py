@@ -1,0 +1,41 @@
+"""The automatic choice of cells per thread of plain FP64 kernels: bit for bit the fields of one
+cell per thread on either side of each of its lines (rows of 160 and 256 cells, launches of 4e6
+and 12e6 cells), with extents that the groups do not divide."""
+import numpy as np
+import pytest
+
+import parallelstencil as ps
+from parallelstencil import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+M64 = __name__ + ".f64"
+ps.init_parallel_stencil(ps.AMDGPU, ps.Float64, 3, module=M64)
+
+
+@pytest.mark.parametrize("shape", [(159, 161, 163), (160, 160, 156), (160, 160, 157), (161, 163, 155), (255, 127, 131),
+                                   (229, 230, 231), (256, 9, 10), (259, 7, 13)])
+def test_automatic_cells_match_one_cell(shape):
+    rng = np.random.default_rng(sum(shape))
+    auto, one = W.define_diffusion3d(False, M64), W.define_diffusion3d(False, M64, cells_x=1, cells_z=1)
+    T, Ci = ps.zeros(*shape), ps.zeros(*shape)
+    T.copy_from(np.asfortranarray(rng.standard_normal(shape)))
+    Ci.copy_from(np.asfortranarray(1.0 + rng.random(shape)))
+    a, b = ps.zeros(*shape), ps.zeros(*shape)
+    for k, T2 in ((auto, a), (one, b)):
+        T2.copy_from(T.to_host())
+        k(T2, T, Ci, 1.3, 1e-3, 0.1, 0.2, 0.3)
+    assert np.array_equal(a.to_host().view(np.uint64), b.to_host().view(np.uint64)), shape
+    nx, ny, nz = (n - 1 for n in shape)  # staggered arrays: the launch box is the largest of them
+    F = [(rng.standard_normal(s)) for s in ((nx + 1, ny, nz), (nx, ny + 1, nz), (nx, ny, nz + 1), (nx, ny, nz))]
+    out = []
+    for kw in ({}, dict(cells_x=1, cells_z=1)):
+        V, P = W.define_acoustic3d(M64, **kw)
+        D = [ps.zeros(*f.shape) for f in F]
+        for d, f in zip(D, F):
+            d.copy_from(np.asfortranarray(f))
+        V(*D, 1e-2, 1.1, 0.1, 0.2, 0.3)
+        P(D[3], D[0], D[1], D[2], 1e-2, 1.2, 0.1, 0.2, 0.3)
+        out.append([np.ascontiguousarray(d.to_host()).view(np.uint64) for d in D])
+    for x, y in zip(*out):
+        assert np.array_equal(x, y), shape
