@@ -193,7 +193,6 @@ __global__ void __launch_bounds__(256) nn_gemm_k(int M, int N, int K, const bf16
 // With C below 8 (VEC false) the k of one 16-byte piece cross taps: the lane collects its 8 values
 // one by one from the patch.
 constexpr int KS = 64;
-constexpr int KD = 2;  // weight stages in flight ahead of the one in LDS (even: stage s goes through LDS buffer s & 1)
 
 __device__ __forceinline__ unsigned fdiv(unsigned e, unsigned d, unsigned magic) { return d == 1u ? e : __umulhi(e, magic); }
 
@@ -221,6 +220,11 @@ __global__ void __launch_bounds__(64 * WM * WN) nn_conv3_k(const bf16_t* __restr
                                                            unsigned pmagic) {
   constexpr bool VEC = MODE != 0;
   constexpr int NTH = 64 * WM * WN, NB = 16 * NT * WN, LDB = NB + 8;
+  // weight stages in flight ahead of the one in LDS (even: stage s goes through LDS buffer s & 1): 4 for the
+  // tiles of the long sums, where one workgroup is on a CU and little hides a miss (256 -> 256 at 64^2 18.9
+  // -> 17.8 us, 8 x 32^2 384 -> 128 27.0 -> 25.5); 256 x 32, two workgroups on a CU, is better off with 2
+  // (64 -> 64 at 256^2 12.4 us, 12.7 with 4)
+  constexpr int KD = MODE == 2 && !(MT == 2 && NT == 2 && WM == 8) ? 4 : 2;
   constexpr int PIECES = KS * NB / 8, PB = (PIECES + NTH - 1) / NTH;  // 16-byte pieces of a weight stage, and per thread
   extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
   bf16_t* const Bs = lds;
@@ -424,7 +428,7 @@ __global__ void __launch_bounds__(64 * WM * WN) nn_conv3_k(const bf16_t* __restr
 // workgroups of one 64 x 64 tile each, and spent 32 of its 64 columns on padding.
 constexpr int WGS = 40;  // LDS elements per pixel: 32 channels, 16 bytes of padding against bank conflicts
 
-template <bool VEC>
+template <bool VX, bool VD>  // rows of x, of dy are whole aligned 16-byte pieces
 __global__ void __launch_bounds__(512, 2) nn_conv3_wgrad_k(const bf16_t* __restrict__ x, int H, int W, int C, const bf16_t* __restrict__ dy,
                                                            long long sbk, int N, float* __restrict__ gw, long long ldc, int lgTX, int tilesx,
                                                            int tilesy, int ntiles, unsigned pmagic) {
@@ -447,7 +451,7 @@ __global__ void __launch_bounds__(512, 2) nn_conv3_wgrad_k(const bf16_t* __restr
       rx[j] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
       if (p < (unsigned)npx && (unsigned)yy < (unsigned)H && (unsigned)xx < (unsigned)W) {
         const bf16_t* const src = x + (pb + (long long)yy * W + xx) * C + c;
-        if (VEC) {
+        if (VX) {
           if (c < C) rx[j] = *(const s16x8*)src;
         } else {
           for (int i = 0; i < 8; ++i)
@@ -461,7 +465,7 @@ __global__ void __launch_bounds__(512, 2) nn_conv3_wgrad_k(const bf16_t* __restr
       rd[j] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
       if (yy < H && xx < W) {
         const bf16_t* const src = dy + (pb + (long long)yy * W + xx) * sbk + n;
-        if (VEC) {
+        if (VD) {
           if (n < N) rd[j] = *(const s16x8*)src;
         } else {
           for (int i = 0; i < 8; ++i)
@@ -1016,9 +1020,15 @@ int wgrad_launch(int N, long long K, const bf16_t* x, int H, int W, int C, const
   const int S = (int)std::min<long long>(std::min<long long>(nt, 65535), std::max<long long>(1, want / (gc * gn)));
   const unsigned pmagic = (unsigned)((0x100000000ULL + tx + 1) / (tx + 2));
   const dim3 grid((unsigned)gc, (unsigned)gn, (unsigned)S);
-  const bool v = C % 8 == 0 && N % 8 == 0 && sbk % 8 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)dy & 15) == 0;
-  if (v) hipLaunchKernelGGL((nn_conv3_wgrad_k<true>), grid, dim3(512), 0, st, x, H, W, C, dy, sbk, N, (float*)gw, ldc, lg, tilesx, tilesy, (int)nt, pmagic);
-  else hipLaunchKernelGGL((nn_conv3_wgrad_k<false>), grid, dim3(512), 0, st, x, H, W, C, dy, sbk, N, (float*)gw, ldc, lg, tilesx, tilesy, (int)nt, pmagic);
+  // the first layer's few input channels come one by one, its dy in whole pieces all the same
+  const bool vx = C % 8 == 0 && ((uintptr_t)x & 15) == 0, vd = N % 8 == 0 && sbk % 8 == 0 && ((uintptr_t)dy & 15) == 0;
+#define NN_WGRAD(VX, VD) \
+  hipLaunchKernelGGL((nn_conv3_wgrad_k<VX, VD>), grid, dim3(512), 0, st, x, H, W, C, dy, sbk, N, (float*)gw, ldc, lg, tilesx, tilesy, (int)nt, pmagic)
+  if (vx && vd) NN_WGRAD(true, true);
+  else if (vx) NN_WGRAD(true, false);
+  else if (vd) NN_WGRAD(false, true);
+  else NN_WGRAD(false, false);
+#undef NN_WGRAD
   return launched("ps_nn_gemm_im2col");
 }
 

@@ -21,7 +21,7 @@ def _bf(a):
 # image sizes around the 8- and 16-column tiles, channels around the groups of 8 and 32 and beyond what
 # fits two patches (and one patch) into LDS, output channels around 32 and 64
 CONV = [(1, 1, 1, 8, 8), (2, 15, 17, 32, 33), (1, 16, 16, 24, 31), (3, 9, 8, 40, 65), (1, 33, 31, 7, 4), (2, 20, 24, 128, 130), (1, 70, 70, 96, 32),
-        (4, 64, 64, 192, 64), (1, 10, 40, 384, 96), (1, 12, 12, 512, 16), (1, 300, 260, 32, 32), (2, 5, 100, 9, 12), (1, 17, 130, 2, 3)]
+        (4, 64, 64, 192, 64), (1, 10, 40, 384, 96), (1, 12, 12, 512, 16), (1, 300, 260, 32, 32), (2, 5, 100, 9, 12), (1, 17, 130, 2, 3), (2, 21, 37, 3, 40)]
 
 
 @pytest.mark.parametrize("B,H,W,C,N", CONV)
