@@ -2866,6 +2866,23 @@ int idx_span(const Kernel& K, int q) {
   return (int)span;
 }
 
+bool only_writes(const Kernel& K) {
+  std::function<bool(const NodeP&)> reads = [&](const NodeP& n) -> bool {
+    if (!n) return false;
+    if (n->k == NK::Index) return true;
+    if (array_assign(n)) {  // the target itself is a write, a compound one also a read
+      if (!n->s.empty()) return true;
+      for (size_t i = 1; i < n->a[0]->a.size(); ++i)
+        if (reads(n->a[0]->a[i])) return true;
+      return reads(n->a[1]);
+    }
+    for (auto& a : n->a)
+      if (reads(a)) return true;
+    return false;
+  };
+  return K.body && !reads(K.body);
+}
+
 Emitted lower_kernel(const Kernel& k, const std::vector<ArgKind>& kinds, const Variant& v) {
   Emitter e(k, kinds, v);
   return e.run();

@@ -215,6 +215,9 @@ bool groupable_body(const Kernel& k, bool z = false);
 // Largest spread of offsets along dimension q (0 x, 2 z) with which the kernel body accesses one
 // array (0: no neighbours along q).
 int idx_span(const Kernel& k, int q);
+
+// Whether no statement of the body reads an array element (array assignments and their conditions).
+bool only_writes(const Kernel& k);
 std::string kernel_info_json(const Kernel& k);
 
 // Bounds proof: true if every array access of the kernel stays inside its

@@ -39,3 +39,31 @@ def test_automatic_cells_match_one_cell(shape):
         out.append([np.ascontiguousarray(d.to_host()).view(np.uint64) for d in D])
     for x, y in zip(*out):
         assert np.array_equal(x, y), shape
+
+
+WRITES = """
+@parallel_indices (ix, iy, iz) function writes!(A, B, C, s::Data.Number)
+    if ix >= 2 && ix <= size(A, 1) - 1 && iz >= 2 && iz <= size(A, 3) - 1
+        A[ix, iy, iz] = 0.0
+        B[ix, iy, iz] = s * 0.5 + ix
+    end
+    C[ix, iy, iz] = s
+    return
+end
+"""
+READS = WRITES.replace("C[ix, iy, iz] = s\n", "C[ix, iy, iz] += s\n")
+
+
+@pytest.mark.parametrize("src", [WRITES, READS])
+@pytest.mark.parametrize("shape", [(2, 3, 8), (7, 5, 9), (64, 33, 10), (130, 17, 7), (259, 20, 31)])
+def test_kernels_without_reads_match_one_cell(src, shape):
+    # four z cells per thread where nothing is read; sizes that neither 4 z cells nor the block divide
+    out = []
+    for kw in ({}, dict(cells_x=1, cells_z=1)):
+        k = ps.core._define("parallel_indices", src, kw, M64)
+        D = [ps.fill(0.25 * i, *shape) for i in range(3)]
+        for _ in range(2):
+            k(*D, 1.75)
+        out.append([np.ascontiguousarray(d.to_host()).view(np.uint64) for d in D])
+    for x, y in zip(*out):
+        assert np.array_equal(x, y), shape
