@@ -33,8 +33,9 @@ int ps_nn_gemm(int M, int N, int K, const void* A, int64_t sam, int64_t sak, con
 
 /* ps_nn_gemm with A the 3x3 im2col of the NHWC input x (ps_nn_im2col's col, never stored):
  * transpose 0: A = col (M = B*H*W pixels, K = 9*C); transpose 1: A = col^T (M = 9*C,
- * K = B*H*W), the weight gradient's operand. Same products in the same order as
- * ps_nn_im2col followed by ps_nn_gemm, so the same results bit for bit. No counterpart in the
+ * K = B*H*W), the weight gradient's operand. transpose 0, and transpose 1 with splitk 1: same
+ * products in the same order as ps_nn_im2col followed by ps_nn_gemm, so the same results bit for
+ * bit; transpose 1 with split K sums pixel tiles (FP32) in an order of its own. No counterpart in the
  * reference (the learned warm start has none); replaces the im2col buffer of the convolutions. */
 int ps_nn_gemm_im2col(int transpose, int M, int N, int K, const void* x, int H, int W, int C, const void* B, int64_t sbk, int64_t sbn,
                       void* Cm, int64_t ldc, const float* bias, int epi, int splitk, void* stream);

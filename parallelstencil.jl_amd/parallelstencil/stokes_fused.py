@@ -1,5 +1,7 @@
 """The pseudo-transient Stokes2D solver of miniapps/Stokes2D.jl with its six launches per iteration
-fused into two, for the launch-bound sizes of the learned warm start (511^2, 1023^2).
+fused into two, and blocks of iterations into launches of several each (ps_stokes2d_iterate, which
+iterates a tile and its halo in LDS; grids of at least 8 x 8), for the launch-bound sizes of the
+learned warm start (511^2, 1023^2).
 
 One PT iteration of the miniapp (:111-116) is compute_P!, compute_τ!, compute_dV!, compute_V!,
 bc_y!(Vx), bc_x!(Vy). Here:
