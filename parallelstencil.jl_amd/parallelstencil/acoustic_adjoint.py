@@ -153,27 +153,52 @@ class Acoustic2DInversion:
         self.snap = [(z(nx + 1, ny), z(nx, ny + 1)) for _ in range(self.seg)]
         # numbertype scalars
         self._t = np.float32 if core._numbertype_of(module) == core.Float32 else np.float64
-        self._plans = {}  # prepared launches by step and default stream
+        self._plans = {}  # group -> (what its launches are bound to, {(step, default stream): prepared launch})
 
-    def _run(self, key, make):
-        """Runs the prepared launch `key` of the current default stream, made by make() on first use: a
-        step of this model takes a few microseconds, less than building its argument blocks anew."""
-        key = (key, core._stream_handle(None))
-        L = self._plans.get(key)
+    def _follow(self):
+        """Drops the prepared launches bound to anything that has changed since they were made: the scalars
+        of the setup, the source samples (by value: they may be written in place), the kernels and the
+        arrays. Called at the start of every run, so a launch never outlives the values it holds."""
+        s, t = self.s, self._t
+        bits = lambda *v: np.array([t(x) for x in v]).tobytes()  # noqa: E731
+        state, adj = (self.P, self.Vx, self.Vy), (self.lP, self.lVx, self.lVy)
+        line = (s.rx0, s.rdx, s.ry, s.nrec)
+        now = {
+            "V": (self.k_v, state, bits(s.dt, s.rho, s.dx, s.dy)),
+            "P": (self.k_p, state, self.K, bits(s.dt, s.dx, s.dy)),
+            "inject": (self.k_inj, self.P, s.isx, s.isy, bits(*(s.src[n] for n in range(s.nt)))),
+            "record": (self.k_rec, self.D, self.P, line),
+            "residual": (self.k_res, self.lP, self.D, self.Dobs, line),
+            "K": (self.k_gk, self.gK, self.lP, tuple(A for pair in self.snap for A in pair), bits(s.dt, s.dx, s.dy)),
+            "lV": (self.k_av, adj, self.K, bits(s.dt, s.dx, s.dy)),
+            "lP": (self.k_ap, adj, bits(s.dt, s.rho, s.dx, s.dy)),
+        }
+        for group, bound in now.items():
+            if group not in self._plans or self._plans[group][0] != bound:
+                self._plans[group] = (bound, {})
+
+    def _run(self, group, n, make):
+        """Runs the prepared launch of step n (None: the same for all steps) of `group` on the current
+        default stream, made by make() on first use: a step of this model takes a few microseconds, less than
+        building its argument blocks anew."""
+        plans = self._plans[group][1]
+        key = (n, core._stream_handle(None))
+        L = plans.get(key)
         if L is None:
-            L = self._plans[key] = make()
+            L = plans[key] = make()
         L()
 
     # -------------------------------------------------------------- forward
     def _step(self, n, record=True):
         s, t = self.s, self._t
-        self._run("V", lambda: self.k_v.launcher(self.Vx, self.Vy, self.P, t(s.dt), t(s.rho), t(s.dx), t(s.dy)))
-        self._run("P", lambda: self.k_p.launcher(self.P, self.Vx, self.Vy, self.K, t(s.dt), t(s.dx), t(s.dy)))
-        self._run(("inject", n), lambda: self.k_inj.launcher(self.P, t(s.src[n]), s.isx, s.isy, ranges=((1, 1),)))
+        self._run("V", None, lambda: self.k_v.launcher(self.Vx, self.Vy, self.P, t(s.dt), t(s.rho), t(s.dx), t(s.dy)))
+        self._run("P", None, lambda: self.k_p.launcher(self.P, self.Vx, self.Vy, self.K, t(s.dt), t(s.dx), t(s.dy)))
+        self._run("inject", n, lambda: self.k_inj.launcher(self.P, t(s.src[n]), s.isx, s.isy, ranges=((1, 1),)))
         if record:
-            self._run(("record", n), lambda: self.k_rec.launcher(self.D, self.P, s.rx0, s.rdx, s.ry, n + 1, ranges=((1, s.nrec),)))
+            self._run("record", n, lambda: self.k_rec.launcher(self.D, self.P, s.rx0, s.rdx, s.ry, n + 1, ranges=((1, s.nrec),)))
 
     def _reset_state(self):
+        self._follow()
         for A in (self.P, self.Vx, self.Vy):
             A.fill_(0.0)
 
@@ -217,10 +242,10 @@ class Acoustic2DInversion:
                 self.snap[n - n0][0].copy_(self.Vx, async_=True)
                 self.snap[n - n0][1].copy_(self.Vy, async_=True)
             for n in reversed(range(n0, n1)):
-                self._run(("residual", n), lambda: self.k_res.launcher(self.lP, self.D, self.Dobs, s.rx0, s.rdx, s.ry, n + 1, ranges=((1, s.nrec),)))
-                self._run(("K", n - n0), lambda: self.k_gk.launcher(self.gK, self.lP, *self.snap[n - n0], t(s.dt), t(s.dx), t(s.dy)))
-                self._run("lV", lambda: self.k_av.launcher(self.lVx, self.lVy, self.lP, self.K, t(s.dt), t(s.dx), t(s.dy)))
-                self._run("lP", lambda: self.k_ap.launcher(self.lP, self.lVx, self.lVy, t(s.dt), t(s.rho), t(s.dx), t(s.dy)))
+                self._run("residual", n, lambda: self.k_res.launcher(self.lP, self.D, self.Dobs, s.rx0, s.rdx, s.ry, n + 1, ranges=((1, s.nrec),)))
+                self._run("K", n - n0, lambda: self.k_gk.launcher(self.gK, self.lP, *self.snap[n - n0], t(s.dt), t(s.dx), t(s.dy)))
+                self._run("lV", None, lambda: self.k_av.launcher(self.lVx, self.lVy, self.lP, self.K, t(s.dt), t(s.dx), t(s.dy)))
+                self._run("lP", None, lambda: self.k_ap.launcher(self.lP, self.lVx, self.lVy, t(s.dt), t(s.rho), t(s.dx), t(s.dy)))
         core.synchronize()
         return J, self.gK.to_host().astype(np.float64)
 

@@ -114,3 +114,48 @@ def test_hand_written_adjoint_matches_derivative_kernels():
     assert np.abs(ga).max() > 0
     assert np.abs(ga - g).max() <= 1e-12 * np.abs(g).max()
     assert np.array_equal(Db.to_host(), np.zeros((s.nrec, s.nt)))  # every residual consumed
+
+
+def _same_as_new(inv, s, Dobs, mod, K):
+    """Traces, misfit and gradient of `inv` and of an object made anew from the same setup."""
+    new = AA.Acoustic2DInversion(mod, s, seg=inv.seg)
+    new.set_observed(Dobs)
+    assert np.array_equal(inv.forward(K), new.forward(K))
+    (Ja, ga), (Jb, gb) = inv.gradient(K), new.gradient(K)
+    assert Ja == Jb and np.array_equal(ga, gb)
+    return ga
+
+
+@pytest.mark.parametrize("mod", [MOD64, MOD32])
+def test_changed_setup_is_followed(mod):
+    """One object over several shots: every value of the setup that a step reads may change between two
+    calls, the source samples in place too, and so may the arrays."""
+    s, inv, Dobs = _inv(mod, nx=48, ny=40, nt=40, nrec=8)
+    last = _same_as_new(inv, s, Dobs, mod, s.K)
+
+    def amplify():
+        s.src[3:20] *= 1.5
+
+    def trade():
+        inv.s = AA.Setup(48, 40, 40, seed=9, nrec=8, sigma=9.0)
+
+    changes = [lambda: setattr(s, "isx", s.isx + 3), lambda: setattr(s, "isy", s.isy - 2), lambda: setattr(s, "src", 0.7 * s.src), amplify,
+               lambda: setattr(s, "ry", s.ry - 4), lambda: setattr(s, "rx0", s.rx0 + 1), lambda: setattr(s, "dt", 0.9 * s.dt),
+               lambda: setattr(s, "rho", 1.1), lambda: setattr(s, "dx", 1.05 * s.dx), lambda: setattr(s, "dy", 1.02 * s.dy), trade]
+    for change in changes:
+        change()
+        g = _same_as_new(inv, inv.s, Dobs, mod, s.K)
+        assert not np.array_equal(g, last)
+        last = g
+
+
+def test_changed_arrays_are_followed():
+    s, inv, Dobs = _inv(MOD64, nx=48, ny=40, nt=40, nrec=8)
+    inv.gradient(s.K)
+    old = inv.K
+    for name in ("K", "D", "Dobs", "P", "Vx", "Vy", "lP", "lVx", "lVy", "gK"):
+        setattr(inv, name, ps.zeros(*getattr(inv, name).shape))
+    inv.snap = [tuple(ps.zeros(*A.shape) for A in pair) for pair in inv.snap]
+    inv.set_observed(Dobs)
+    old.fill_(7.0)  # nothing reads the array that was replaced
+    _same_as_new(inv, s, Dobs, MOD64, s.K)
