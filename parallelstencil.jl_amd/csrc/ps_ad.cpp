@@ -107,8 +107,8 @@ bool flat_function(const std::string& f) {
 
 class Ad {
  public:
-  Ad(const Kernel& K, bool reverse, const std::map<std::string, std::string>& annot, const std::string& form = "scatter")
-      : K(K), reverse(reverse), form(form) {
+  Ad(const Kernel& K, bool reverse, const std::map<std::string, std::string>& annot, const std::string& form, bool gather_factors)
+      : K(K), reverse(reverse), form(form), gather_factors(gather_factors && K.opt.numbertype == "Float64") {
     for (auto& p : K.def.params) {
       auto it = annot.find(p.name);
       if (it == annot.end() || it->second == "Const") continue;
@@ -179,6 +179,7 @@ class Ad {
   const Kernel& K;
   bool reverse;
   std::string form;                           // scatter | gather | clear
+  bool gather_factors;                        // gathered() rewrites
   bool no_temps = false;                      // contributions as pure expressions (gather form)
   std::map<std::string, std::string> shadow;  // duplicated argument -> shadow parameter
   std::set<std::string> noneed;               // DuplicatedNoNeed arguments
@@ -850,8 +851,12 @@ class Ad {
   // expression of scalar arguments and literals (which the host evaluates once per launch), terms with
   // the same loads merged. The chain rule leaves (((-((g*(dt/Cp))/dx))/dx)*(-lam)) and sums of six of
   // them at a cell; gathered they are one load product times one number. The quantity is the same up to
-  // the rounding of the factors, whose order is this transformation's own. An expression with a
-  // comparison among its factors (Bool * x is a strong zero) is left as it is.
+  // the rounding of the factors, whose order is this transformation's own, while the product of the factors
+  // alone and that of the loads stay within the type's range. Float64's 1e+-308 leaves room for that;
+  // Float32's 1e+-38 does not (lam = 1e15 over dx^2 of dx = 1e-13 is 1e41, times a seed of 1e-25 it is
+  // 1e16), so only kernels of number type Float64 are rewritten (Float32 gather kernel at 256^3: 87 us
+  // without, 80 with it). An expression with a comparison among its factors (Bool * x is a strong zero) is
+  // left as it is, and a launch with a Bool scalar takes the kernel without this.
   bool uniform(const NodeP& n) const {
     if (n->k == NK::Num) return true;
     if (n->k == NK::Ident) {
@@ -899,7 +904,7 @@ class Ad {
   }
   NodeP gathered(const NodeP& e) const {
     std::vector<Term> ts;
-    if (!terms(e, false, ts)) return e;
+    if (!gather_factors || !terms(e, false, ts)) return e;
     std::vector<std::string> order;
     std::map<std::string, std::vector<Term>> groups;
     for (auto& t : ts) {
@@ -1084,7 +1089,7 @@ class Ad {
 
 }  // namespace
 
-Kernel derivative_kernel(const Kernel& K, const JVal& spec) {
+Kernel derivative_kernel(const Kernel& K, const JVal& spec, bool gather_factors) {
   std::string mode = "Reverse";
   if (auto* m = spec.get("mode")) mode = m->s;
   if (mode.rfind("Enzyme.", 0) == 0) mode = mode.substr(7);
@@ -1106,7 +1111,7 @@ Kernel derivative_kernel(const Kernel& K, const JVal& spec) {
   if (auto* f = spec.get("form")) form = f->s;
   if (form != "scatter" && form != "gather" && form != "clear")
     throw PsError(PS_EARGUMENT, "∇: unknown derivative form '" + form + "' (scatter, gather or clear)");
-  return Ad(K, mode == "Reverse", annot, form).run();
+  return Ad(K, mode == "Reverse", annot, form, gather_factors).run();
 }
 
 }  // namespace ps

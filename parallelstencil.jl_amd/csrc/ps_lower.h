@@ -204,8 +204,9 @@ NodeP canonical_indices(const NodeP& n);
 // "form": "scatter"|"gather"|"clear"}; the derivative takes the primal's parameters followed by
 // one shadow per duplicated array. Reverse mode of @parallel kernels also has a two-kernel form:
 // "gather" (each point sums the adjoints that reach it) then "clear" (seeds and kept primal
-// updates); it raises an ArgumentError where it does not apply.
-Kernel derivative_kernel(const Kernel& k, const JVal& spec);
+// updates); it raises an ArgumentError where it does not apply. gather_factors: whether the gather
+// form may gather the uniform factors of its terms (not for launches with a Bool scalar).
+Kernel derivative_kernel(const Kernel& k, const JVal& spec, bool gather_factors = true);
 Emitted lower_kernel(const Kernel& k, const std::vector<ArgKind>& kinds, const Variant& v);
 // Whether a plain kernel's body can run as groups of cells (Variant::cx, Variant::cz): a sequence
 // of array assignments, each optionally under an if without else whose condition bounds the x

@@ -15,6 +15,7 @@
 #include <cstring>
 #include <dlfcn.h>
 #include <fstream>
+#include <functional>
 #include <map>
 #include <memory>
 #include <unordered_map>
@@ -272,7 +273,8 @@ struct Module {
 struct LaunchEntry;
 
 struct KernelObj {
-  Kernel K;
+  const std::shared_ptr<Kernel> kernel = std::make_shared<Kernel>();  // shared with the derivatives made from it
+  Kernel& K = *kernel;
   std::mutex mu;
   std::map<std::string, std::shared_ptr<Module>> variants;  // key: kinds+variant
   // launch plans (geometry, variant, module) by argument signature: repeated launches of the
@@ -284,6 +286,9 @@ struct KernelObj {
   std::map<std::string, std::shared_ptr<Kernel>> padspec;
 };
 
+  // gather form of a derivative: the kernel without gathered factors, for launches with a Bool scalar
+  std::function<Kernel()> make_ungathered;
+  std::shared_ptr<Kernel> ungathered;
 struct State {
   std::mutex mu;
   bool inited = false;
@@ -503,9 +508,19 @@ std::string kinds_key(const std::vector<ArgKind>& k) {
 
 // The kernel a launch with these arguments runs: the definition itself, or for padding=true
 // kernels whose indices compare parent sizes, its specialisation to the arguments' parents
+// The kernel before any specialisation: that without gathered factors where a scalar is a Bool.
+const Kernel& base_kernel(KernelObj* ko, const ps_arg* args, int nargs) {
+  bool bools = false;
+  for (int i = 0; i < nargs && ko->make_ungathered; ++i) bools = bools || (args[i].kind == PS_ARG_SCALAR && args[i].dtype == PS_BOOL);
+  if (!bools) return ko->K;
+  std::lock_guard<std::mutex> lk(ko->pmu);
+  if (!ko->ungathered) ko->ungathered = std::make_shared<Kernel>(ko->make_ungathered());
+  return *ko->ungathered;
+}
+
 // (*bits receives the comparison results, "" when there are none).
 const Kernel& kernel_for(KernelObj* ko, const ps_arg* args, int nargs, std::string* bits) {
-  const Kernel& K = ko->K;
+  const Kernel& K = base_kernel(ko, args, nargs);
   bits->clear();
   if (K.pgt_terms.empty()) return K;
   for (auto& t : K.pgt_terms) {
@@ -514,7 +529,7 @@ const Kernel& kernel_for(KernelObj* ko, const ps_arg* args, int nargs, std::stri
     bits->push_back(pdim(args[t[0]].field, t[2] - 1) > pdim(args[t[1]].field, t[2] - 1) ? '1' : '0');
   }
   std::lock_guard<std::mutex> lk(ko->pmu);
-  auto& slot = ko->padspec[*bits];
+  auto& slot = ko->padspec[*bits + (&K == &ko->K ? "" : "u")];
   if (!slot) slot = std::make_shared<Kernel>(specialize_padding(K, *bits));
   return *slot;
 }
@@ -1217,7 +1232,11 @@ extern "C" int ps_kernel_derivative(ps_kernel primal, const char* spec_json, ps_
   if (!p || !out) throw PsError(PS_EARGUMENT, "ps_kernel_derivative: null kernel");
   auto ko = new KernelObj();
   try {
-    ko->K = derivative_kernel(p->K, json_parse(spec_json ? spec_json : ""));
+    const JVal spec = json_parse(spec_json ? spec_json : "");
+    ko->K = derivative_kernel(p->K, spec);
+    const JVal* form = spec.get("form");
+    if (form && form->s == "gather")
+      ko->make_ungathered = [primal = p->kernel, spec] { return derivative_kernel(*primal, spec, false); };
   } catch (...) {
     delete ko;
     throw;
@@ -1375,7 +1394,8 @@ extern "C" int ps_kernel_source(ps_kernel k, const ps_arg* args, int nargs, int 
   KernelObj* ko = (KernelObj*)k;
   Variant v = variant_from_flags(ko->K, flags);
   v.divmode = divmode_of(args, nargs);
-  const Kernel K0 = ko->K.pgt_terms.empty() ? ko->K : specialize_padding(ko->K, std::string(ko->K.pgt_terms.size(), '0'));
+  const Kernel& KB = base_kernel(ko, args, nargs);
+  const Kernel K0 = KB.pgt_terms.empty() ? KB : specialize_padding(KB, std::string(KB.pgt_terms.size(), '0'));
   if (!ko->K.pgt_terms.empty()) v.padbits = std::string(ko->K.pgt_terms.size(), '0');
   Emitted em = lower_kernel(K0, arg_kinds(args, nargs), v);
   if (em.source.size() + 1 > cap) return fail(PS_EARGUMENT, "ps_kernel_source: buffer too small (need " + std::to_string(em.source.size() + 1) + ")");
@@ -1391,9 +1411,9 @@ extern "C" int ps_kernel_precompile(ps_kernel k, const ps_arg* args, int nargs, 
   v.divmode = divmode_of(args, nargs);
   if (!ko->K.pgt_terms.empty()) {
     v.padbits = std::string(ko->K.pgt_terms.size(), '0');
-    get_module(ko, specialize_padding(ko->K, v.padbits), arg_kinds(args, nargs), v, false);
+    get_module(ko, specialize_padding(base_kernel(ko, args, nargs), v.padbits), arg_kinds(args, nargs), v, false);
   } else {
-    get_module(ko, ko->K, arg_kinds(args, nargs), v, false);
+    get_module(ko, base_kernel(ko, args, nargs), arg_kinds(args, nargs), v, false);
   }
   return 0;
   PS_GUARD_END

@@ -555,3 +555,53 @@ def test_memopt_parallel_indices_reverse_both_forms():
         d.use_gather = True
         _close(Ab.to_host(), want)
         assert np.array_equal(A2b.to_host(), np.where(inner, 0.0, y))
+
+
+def _both_forms(k, args, seed, annots):
+    """The shadow of the second argument by the scatter and the gather form, from the same seed of the first."""
+    d = k._derivative("Reverse", annots)
+    assert d._gather is not None
+    outs = []
+    for gather in (False, True):
+        d.use_gather = gather
+        Bb = ps.zeros(*seed.shape, eltype=args[0].eltype).copy_from(np.asfortranarray(seed))
+        Ab = ps.zeros(*seed.shape, eltype=args[0].eltype)
+        k(*args, grad=[(args[0], Bb), (args[1], Ab)])
+        outs.append(Ab.to_host())
+    d.use_gather = True
+    return outs
+
+
+@pytest.mark.parametrize("memopt", [False, True])
+@pytest.mark.parametrize("c,dx,seed", [(1e15, 1e-13, 1e-25), (1e-30, 1e6, 1e30), (1e30, 1e-8, 1e-30), (0.25, 0.1, 1.0)])
+def test_float32_factors_beyond_the_type_alone(memopt, c, dx, seed):
+    """c/dx/dx leaves the range of Float32 (1e41, 1e-42, 1e46), every product with the seed does not: the
+    gather form is as finite and as accurate as the scatter form."""
+    _init(".f32", ps.Float32, 2)
+    k = ps.core._define("parallel", """
+    @parallel function lapdx!(B, A, c, dx)
+        @inn(B) = c*(@d2_xi(A)/dx/dx + @d2_yi(A)/dx/dx)
+        return
+    end""", {"memopt": memopt}, MOD + ".f32")
+    shape = (64, 40)
+    B, A = ps.zeros(*shape, eltype=ps.Float32), ps.zeros(*shape, eltype=ps.Float32)
+    y = ((np.random.default_rng(3).random(shape) + 0.5) * seed).astype(np.float32)
+    scatter, gather = _both_forms(k, (B, A, np.float32(c), np.float32(dx)), y, {"B": "DuplicatedNoNeed", "A": "DuplicatedNoNeed"})
+    assert np.isfinite(scatter).all() and np.abs(scatter).max() > 0
+    # up to 8 terms per cell that cancel, a few roundings each: 32 eps of the largest value
+    assert np.abs(gather - scatter).max() <= 32 * 2.0 ** -23 * np.abs(scatter).max()
+
+
+def test_bool_scalar_stays_a_strong_zero_in_both_forms():
+    """Bool * x is zero for an infinite or NaN x too (Julia's strong zero), also in the gather form."""
+    k = ps.core._define("parallel_indices", """
+    @parallel_indices (ix) function masked!(B, A, m, c)
+        B[ix] = m*A[ix]*c
+        return
+    end""", {}, MOD)
+    y = np.array([1.0, np.inf, -np.inf, np.nan, 2.0])
+    B, A = ps.zeros(5), ps.zeros(5)
+    for m in (False, True):
+        scatter, gather = _both_forms(k, (B, A, m, 3.0), y, {"B": "DuplicatedNoNeed", "A": "DuplicatedNoNeed"})
+        np.testing.assert_array_equal(scatter, 3.0 * y if m else np.zeros(5))
+        np.testing.assert_array_equal(gather, scatter)
