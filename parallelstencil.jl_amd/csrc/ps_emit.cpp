@@ -557,6 +557,7 @@ EV Emitter::load(const NodeP& n) {
   bool aff = false;
   std::string ref32;
   std::string off = offset(ai, idx, ic, &aff, &ref32);
+  load_cached = false;  // an index may have been served by the cache
   std::string A = an(ai);
   std::string raw = ref32.empty() ? A + "[" + off + "]" : ref32;
   int dt = kinds[ai].dtype;

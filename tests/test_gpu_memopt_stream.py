@@ -93,3 +93,26 @@ def test_gather_matches_scatter(dims, memopt):
     assert np.array_equal(outs[0][0], outs[1][0])
     # seven products a cell, each a few roundings, in either order: 1e-14 of the largest term (about 5)
     assert np.abs(outs[0][1] - outs[1][1]).max() <= 1e-13
+
+
+INDIRECT = """
+@parallel_indices (ix,iy,iz) function indirect!(B, C, I, s)
+    if (1 < ix < size(B,1) && 1 < iy < size(B,2) && 1 < iz < size(B,3))
+        B[ix,iy,iz] = s/C[ix,iy,iz-1] + s/C[ix,iy,iz+1] + s/C[I[ix,iy,iz],iy,iz]
+    end
+    return
+end
+"""
+
+
+def test_quotient_of_an_element_found_by_an_index_array():
+    # the index is served by a register of the stream, the divisor is not: it is still divided by
+    dims = (64, 20, 70)
+    C = _rand(dims, 1, 0.5)
+    I = ps.zeros(*dims, eltype=ps.Int64).copy_from(np.asfortranarray(np.random.default_rng(2).integers(1, dims[0] + 1, dims)))  # noqa: E741
+    outs = []
+    for memopt in (False, True):
+        B = _rand(dims, 3)
+        ps.core._define("parallel_indices", INDIRECT, {"memopt": memopt, "inbounds": True}, MOD)(B, C, I, 0.7)
+        outs.append(B.to_host())
+    assert np.array_equal(*outs)
