@@ -1,6 +1,6 @@
 """The pseudo-transient Stokes2D solver of miniapps/Stokes2D.jl with its six launches per iteration
 fused into two, and blocks of iterations into launches of several each (ps_stokes2d_iterate, which
-iterates a tile and its halo in LDS; grids of at least 8 x 8), for the launch-bound sizes of the
+iterates a tile and its halo in LDS; grids of 8 to 32768 cells per dimension), for the launch-bound sizes of the
 learned warm start (511^2, 1023^2).
 
 One PT iteration of the miniapp (:111-116) is compute_P!, compute_τ!, compute_dV!, compute_V!,
@@ -30,7 +30,7 @@ import re
 import numpy as np
 
 from . import core
-from ._lib import check, lib, ps_stokes2d
+from ._lib import OutOfMemoryError, check, lib, ps_stokes2d
 from . import workloads as W
 
 STOKES2D_PTAU = """
@@ -92,7 +92,18 @@ class _Iterations:
     """ps_stokes2d_iterate on a solver's fields: several PT iterations per launch. The launches read
     the state from one copy and write the other, so a second copy of the five state arrays is held."""
 
-    MIN = 8  # cells per dimension
+    MIN, MAX = 8, 32768  # cells per dimension that ps_stokes2d_iterate takes
+
+    @classmethod
+    def of(cls, sv, act=None):
+        """The iterations of solver `sv`, or None where its two launches serve: grids outside MIN..MAX, and
+        where the device has no memory left for the second copy of the state."""
+        if min(sv.nx, sv.ny) < cls.MIN or max(sv.nx, sv.ny) > cls.MAX:
+            return None
+        try:
+            return cls(sv, act)
+        except OutOfMemoryError:
+            return None
 
     def __init__(self, sv, act=None):
         self.fields = dict(state=(sv.Vx, sv.Vy, sv.Pt, sv.dVxdt, sv.dVydt), coef=(sv.dtPt, sv.Mus, sv.dtVx, sv.dtVy, sv.Rog),
@@ -151,7 +162,7 @@ class Stokes2DFused:
             self.k_dvv.launcher(self.Rx, self.Ry, self.dVxdt, self.dVydt, self.Vx, self.Vy, self.Pt, self.Rog, self.txx, self.tyy,
                                 self.txy, self.dtVx, self.dtVy, self.dampX, self.dampY, self.dx, self.dy, ranges=rng),
         ]
-        self._many = _Iterations(self) if min(nx, ny) >= _Iterations.MIN else None
+        self._many = _Iterations.of(self)
         self._graph = None
         self._host_err = np.zeros(4)
         self.iterate(1)  # compiles and loads both kernels (zero fields stay zero)
@@ -184,7 +195,7 @@ class Stokes2DFused:
 
     def iterate(self, n):
         """n PT iterations (miniapps/Stokes2D.jl:111-116), asynchronous: several per launch, a single
-        one by the two kernels above."""
+        one (and all on the grids that _Iterations leaves to them) by the two kernels above."""
         if n > 1 and self._many is not None:
             self._many(n)
             return
@@ -327,7 +338,7 @@ class Stokes2DBatch:
             self.k_dvv.launcher(self.Act, self.Rx, self.Ry, self.dVxdt, self.dVydt, self.Vx, self.Vy, self.Pt, self.Rog, self.txx,
                                 self.tyy, self.txy, self.dtVx, self.dtVy, self.dampX, self.dampY, self.dx, self.dy, ranges=rng),
         ]
-        self._many = _Iterations(self, self.Act) if min(nx, ny) >= _Iterations.MIN else None
+        self._many = _Iterations.of(self, self.Act)
         self._graph = None
         self.iterate(1)  # compiles and loads both kernels (no plane is active yet)
         self._check()

@@ -104,3 +104,53 @@ def test_plane_reductions_match_the_views(shapes):
         want = [a.view((1, 1, s + 1), (a.shape[0], a.shape[1], s + 1)).reduce(op) for s in range(planes) for a in A]
         assert np.array_equal(out.to_host(), want), op
     assert lib.ps_plane_reduce_noalloc(*args(0, need - 1)) == -1
+
+
+@pytest.mark.parametrize("nx,ny", [(40000, 12), (9, 33000)])
+def test_grids_beyond_the_tiles_take_the_two_launches(nx, ny):
+    # more than 32768 cells in a dimension: ps_stokes2d_iterate refuses them, the solver does not
+    a, b = (F.Stokes2DFused(MOD, nx, ny, nout=4) for _ in range(2))
+    for sv in (a, b):
+        _start(sv, 3)
+    a.iterate_block()
+    for _ in range(4):
+        b.iterate(1)
+    ps.synchronize()
+    assert np.isfinite(a.error())
+    for k in FIELDS:
+        assert np.array_equal(_bits(getattr(a, k)), _bits(getattr(b, k))), k
+
+
+@pytest.mark.parametrize("batch", [False, True])
+def test_without_memory_for_a_second_state(batch, monkeypatch):
+    """The second copy of the state is what the blocks of iterations need beyond the solver's arrays: where it
+    cannot be had the solver iterates by the two launches."""
+    zeros = F.core.zeros
+    left = [0]
+
+    def scarce(*shape, **kw):
+        left[0] -= 1
+        if left[0] < 0:
+            raise ps.OutOfMemoryError("device memory")
+        return zeros(*shape, **kw)
+
+    make = lambda: F.Stokes2DBatch(MOD, 20, 18, 3, graph=False) if batch else F.Stokes2DFused(MOD, 20, 18, graph=False)  # noqa: E731
+    count = [0]
+    monkeypatch.setattr(F.core, "zeros", lambda *s, **kw: (count.__setitem__(0, count[0] + 1), zeros(*s, **kw))[1])
+    b = make()
+    _start(b, 5)
+    left[0] = count[0] - 1  # the last array of the second state fails
+    monkeypatch.setattr(F.core, "zeros", scarce)
+    a = make()
+    monkeypatch.undo()
+    assert b._many is not None and a._many is None
+    _start(a, 5)
+    if batch:
+        for sv in (a, b):
+            for s in range(3):
+                sv.set_active(s, True)
+    a.iterate(7)
+    b.iterate(7)
+    ps.synchronize()
+    for k in FIELDS:
+        assert np.array_equal(_bits(getattr(a, k)), _bits(getattr(b, k))), k
