@@ -112,6 +112,12 @@ class _Iterations:
         self.act = act
         self.q = ps_stokes2d(dx=sv.dx, dy=sv.dy, dampX=sv.dampX, dampY=sv.dampY)
         self.stream = core._stream_handle(None)
+        # fewest iterations worth a call. The state returns to its own arrays after an even number of
+        # launches, so 2 or 3 iterations come to launches of 1 and 2, each of which reads and writes all
+        # fields and computes a halo. Where the tiles fill the GPU (more than 256 of 24 x 24 cells) that is
+        # slower than the two launches: 1023^2 54 us an iteration against 37 with n = 2, 39 against 37 with
+        # n = 3, 32 with n = 4; 511^2 16, 12 and 9 against 12.5; at 255^2 n = 2 takes 9.9 against 10.4.
+        self.least = 4 if -(-(sv.nx + 1) // 24) * -(-(sv.ny + 1) // 24) * getattr(sv, "S", 1) > 256 else 2
 
     def __call__(self, n):
         for name, arrs in self.fields.items():
@@ -194,9 +200,9 @@ class Stokes2DFused:
             self.Pt.copy_from(Pt)
 
     def iterate(self, n):
-        """n PT iterations (miniapps/Stokes2D.jl:111-116), asynchronous: several per launch, a single
-        one (and all on the grids that _Iterations leaves to them) by the two kernels above."""
-        if n > 1 and self._many is not None:
+        """n PT iterations (miniapps/Stokes2D.jl:111-116), asynchronous: several per launch, or one by one by
+        the two kernels above (few of them, and the grids that _Iterations leaves to them)."""
+        if self._many is not None and n >= self._many.least:
             self._many(n)
             return
         a, b = self._steps
@@ -376,7 +382,7 @@ class Stokes2DBatch:
 
     def iterate(self, n):
         """n PT iterations of every sample, asynchronous."""
-        if n > 1 and self._many is not None:
+        if self._many is not None and n >= self._many.least:
             self._many(n)
             return
         a, b = self._steps

@@ -154,3 +154,17 @@ def test_without_memory_for_a_second_state(batch, monkeypatch):
     ps.synchronize()
     for k in FIELDS:
         assert np.array_equal(_bits(getattr(a, k)), _bits(getattr(b, k))), k
+
+
+@pytest.mark.parametrize("nx,ny,n", [(700, 520, 2), (700, 520, 3), (300, 200, 2), (300, 200, 3)])
+def test_short_blocks(nx, ny, n):
+    # either side of the rule by which 2 and 3 iterations of large grids go by the two launches
+    a, b = (F.Stokes2DFused(MOD, nx, ny, graph=False) for _ in range(2))
+    for sv in (a, b):
+        _start(sv, n)
+    a.iterate(n)
+    for _ in range(n):
+        b.iterate(1)
+    ps.synchronize()
+    for k in FIELDS:
+        assert np.array_equal(_bits(getattr(a, k)), _bits(getattr(b, k))), k
