@@ -284,11 +284,11 @@ struct KernelObj {
   // padding=true kernels comparing parent sizes: the kernel per pattern of comparison results
   std::mutex pmu;
   std::map<std::string, std::shared_ptr<Kernel>> padspec;
-};
-
   // gather form of a derivative: the kernel without gathered factors, for launches with a Bool scalar
   std::function<Kernel()> make_ungathered;
   std::shared_ptr<Kernel> ungathered;
+};
+
 struct State {
   std::mutex mu;
   bool inited = false;
@@ -506,8 +506,6 @@ std::string kinds_key(const std::vector<ArgKind>& k) {
   return s;
 }
 
-// The kernel a launch with these arguments runs: the definition itself, or for padding=true
-// kernels whose indices compare parent sizes, its specialisation to the arguments' parents
 // The kernel before any specialisation: that without gathered factors where a scalar is a Bool.
 const Kernel& base_kernel(KernelObj* ko, const ps_arg* args, int nargs) {
   bool bools = false;
@@ -518,6 +516,8 @@ const Kernel& base_kernel(KernelObj* ko, const ps_arg* args, int nargs) {
   return *ko->ungathered;
 }
 
+// The kernel a launch with these arguments runs: the definition itself, or for padding=true
+// kernels whose indices compare parent sizes, its specialisation to the arguments' parents
 // (*bits receives the comparison results, "" when there are none).
 const Kernel& kernel_for(KernelObj* ko, const ps_arg* args, int nargs, std::string* bits) {
   const Kernel& K = base_kernel(ko, args, nargs);
