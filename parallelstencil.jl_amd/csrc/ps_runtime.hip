@@ -28,6 +28,7 @@
 
 #include "ps_amd.h"
 #include "ps_lower.h"
+#include "ps_transfer.h"
 
 using namespace ps;
 
@@ -648,31 +649,81 @@ extern "C" int ps_device_sync(void) {
   return check_err_flag(S().stream0);
 }
 
-// Transfers of fields whose rows are not dense go through a dense block on the device, packed or
-// unpacked by a kernel: a strided copy moves its rows one by one, about 9 us each (64^3 FP64 37 ms,
-// 256^3 604 ms to the device; through the block 0.08 and 4.7). The block is shared by all transfers (each holds the
-// lock until its stream is done with it), at most kStageMax large, larger fields pass it in pieces; it is
-// released with the last field.
-constexpr size_t kStageMax = 32u << 20;
-struct Stage {
-  std::mutex mu;
-  char* p = nullptr;
-  size_t cap = 0;
-  std::atomic<int64_t> fields{0};  // live allocations of fields
+// Rows of w elements of T between a field (row r is row r % ny of plane r / ny) and a dense block
+template <class T, bool TO_FIELD>
+__global__ void __launch_bounds__(256) ps_rows_k(T* __restrict__ field, long long w, long long ny, long long pitch, long long plane,
+                                                 long long row0, long long rows, T* __restrict__ dense) {
+  for (long long r = blockIdx.y; r < rows; r += gridDim.y) {
+    const long long z = (row0 + r) / ny, y = (row0 + r) - z * ny;
+    T* const f = field + y * pitch + z * plane;
+    T* const d = dense + r * w;
+    for (long long x = (long long)blockIdx.x * 256 + threadIdx.x; x < w; x += (long long)gridDim.x * 256) {
+      if (TO_FIELD) f[x] = d[x];
+      else d[x] = f[x];
+    }
+  }
+}
+
+namespace {
+
+// One transfer between a field and host memory on a stream, for ps_transfer.h.
+struct Transfer {
+  const ps_field& f;
+  hipStream_t st;
+  bool to_field;
+
+  static char* alloc(size_t n) {
+    char* p = nullptr;
+    if (hipMalloc((void**)&p, n) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  static void free(char* p) { (void)hipFree(p); }
+  int copy(char* dev, char* h, size_t n) {
+    return done(to_field ? hipMemcpyAsync(dev, h, n, hipMemcpyHostToDevice, st) : hipMemcpyAsync(h, dev, n, hipMemcpyDeviceToHost, st));
+  }
+  int sync() { return done(hipStreamSynchronize(st)); }
+  char* row(int64_t r) const { return (char*)f.ptr + ((r % f.dims[1]) * f.pitch + (r / f.dims[1]) * f.plane) * (int64_t)elsize(f.dtype); }
+  int rows(char* block, int64_t r, int64_t n) {
+    switch (elsize(f.dtype)) {
+      case 8: return rows_of<uint64_t>(block, r, n);
+      case 4: return rows_of<uint32_t>(block, r, n);
+      case 2: return rows_of<uint16_t>(block, r, n);
+      default: return rows_of<uint8_t>(block, r, n);
+    }
+  }
+
+ private:
+  template <class T>
+  int rows_of(char* block, int64_t r, int64_t n) {
+    const dim3 grid((unsigned)std::min<int64_t>((f.dims[0] + 255) / 256, 1024), (unsigned)std::min<int64_t>(n, 32768));
+    auto k = to_field ? ps_rows_k<T, true> : ps_rows_k<T, false>;
+    hipLaunchKernelGGL(k, grid, dim3(256), 0, st, (T*)f.ptr, (long long)f.dims[0], (long long)f.dims[1], (long long)f.pitch, (long long)f.plane, (long long)r,
+                       (long long)n, (T*)block);
+    return done(hipGetLastError());
+  }
+  static int done(hipError_t e) { return e == hipSuccess ? 0 : fail(PS_EHIP, std::string("field transfer: ") + hipGetErrorString(e)); }
 };
-static Stage& stage() {
-  static Stage s;
-  return s;
+
+BlockPool<Transfer>& block_pool() {
+  static BlockPool<Transfer>& p = *new BlockPool<Transfer>;  // outlives the fields a program frees at its end
+  return p;
 }
-static void stage_released(int64_t left) {
-  if (left > 0) return;
-  Stage& g = stage();
-  std::lock_guard<std::mutex> lk(g.mu);
-  if (g.fields.load() > 0 || !g.p) return;
-  (void)hipFree(g.p);
-  g.p = nullptr;
-  g.cap = 0;
+
+int transfer(const ps_field& f, char* host, hipStream_t st, bool to_field) {
+  const size_t w = (size_t)f.dims[0] * elsize(f.dtype);
+  const int64_t rows = f.dims[1] * f.dims[2];
+  if (w == 0 || rows == 0) return 0;
+  if (!f.ptr || !host) return fail(PS_EHIP, "invalid argument: a transfer needs device and host memory");
+  Transfer t{f, st, to_field};
+  if ((f.dims[1] == 1 || f.pitch == f.dims[0]) && (f.dims[2] == 1 || f.plane == f.dims[0] * f.dims[1])) {  // dense
+    const int rc = t.copy((char*)f.ptr, host, w * (size_t)rows);
+    return rc ? rc : t.sync();
+  }
+  return transfer_rows(t, block_pool(), to_field, w, rows, host);
 }
+
+}  // namespace
 
 // ---------------------------------------------------------------------------
 // fields
@@ -721,7 +772,7 @@ extern "C" int ps_field_alloc(int ndims, const int64_t dims[3], int dtype, ps_fi
   out->dtype = dtype;
   out->ndims = ndims;
   out->alloc_bytes = bytes;
-  ++stage().fields;
+  block_pool().field_made();
   return 0;
 }
 
@@ -765,7 +816,7 @@ extern "C" int ps_cellarray_alloc(int ndims, const int64_t dims[3], int cellndim
   out->dtype = dtype;
   out->ndims = ndims;
   out->alloc_bytes = bytes;
-  ++stage().fields;
+  block_pool().field_made();
   out->ncomp = (int32_t)nc;
   for (int i = 0; i < 4; ++i) out->celldims[i] = cd[i];
   out->blocklen = B;
@@ -778,7 +829,7 @@ extern "C" int ps_field_free(ps_field* f) {
   PS_HIP(hipFree(f->base));
   f->base = nullptr;
   f->ptr = nullptr;
-  stage_released(--stage().fields);
+  block_pool().field_freed();
   return 0;
 }
 
@@ -799,80 +850,14 @@ extern "C" int ps_field_view(const ps_field* parent, const int64_t lo[3], const 
   return 0;
 }
 
-// Rows of w elements of T between a field (row r is row r % ny of plane r / ny) and a dense block
-template <class T, bool TO_FIELD>
-__global__ void __launch_bounds__(256) ps_rows_k(T* __restrict__ field, long long w, long long ny, long long pitch, long long plane,
-                                                 long long row0, long long rows, T* __restrict__ dense) {
-  for (long long r = blockIdx.y; r < rows; r += gridDim.y) {
-    const long long z = (row0 + r) / ny, y = (row0 + r) - z * ny;
-    T* const f = field + y * pitch + z * plane;
-    T* const d = dense + r * w;
-    for (long long x = (long long)blockIdx.x * 256 + threadIdx.x; x < w; x += (long long)gridDim.x * 256) {
-      if (TO_FIELD) f[x] = d[x];
-      else d[x] = f[x];
-    }
-  }
-}
-
-template <bool TO_FIELD>
-static int transfer(const ps_field& f, char* host, hipStream_t st) {
-  const size_t es = elsize(f.dtype), w = (size_t)f.dims[0] * es;
-  const int64_t rows = f.dims[1] * f.dims[2];
-  if (w == 0 || rows == 0) return 0;
-  if (!f.ptr || !host) return fail(PS_EHIP, "invalid argument: a transfer needs device and host memory");
-  const hipMemcpyKind kind = TO_FIELD ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
-  auto copy = [&](char* dev, char* h, size_t n) { return TO_FIELD ? hipMemcpyAsync(dev, h, n, kind, st) : hipMemcpyAsync(h, dev, n, kind, st); };
-  const bool dense = (f.dims[1] == 1 || f.pitch == f.dims[0]) && (f.dims[2] == 1 || f.plane == f.dims[0] * f.dims[1]);
-  if (dense) {
-    PS_HIP(copy((char*)f.ptr, host, w * (size_t)rows));
-    PS_HIP(hipStreamSynchronize(st));
-    return 0;
-  }
-  if (w > kStageMax) {  // rows worth a copy each
-    for (int64_t r = 0; r < rows; ++r)
-      PS_HIP(copy((char*)f.ptr + ((r % f.dims[1]) * f.pitch + (r / f.dims[1]) * f.plane) * (int64_t)es, host + (size_t)r * w, w));
-    PS_HIP(hipStreamSynchronize(st));
-    return 0;
-  }
-  Stage& g = stage();
-  std::lock_guard<std::mutex> lk(g.mu);
-  const int64_t per = std::min<int64_t>(rows, (int64_t)(kStageMax / w));
-  if (g.cap < w * (size_t)per) {
-    if (g.p) (void)hipFree(g.p);
-    g.p = nullptr;
-    g.cap = 0;
-    if (hipMalloc((void**)&g.p, w * (size_t)per) != hipSuccess) {
-      (void)hipGetLastError();
-      g.p = nullptr;
-      return fail(PS_EOOM, "OutOfMemoryError: cannot allocate " + std::to_string(w * (size_t)per) + " bytes of device memory for a transfer");
-    }
-    g.cap = w * (size_t)per;
-  }
-  for (int64_t r = 0; r < rows; r += per) {
-    const int64_t n = std::min(per, rows - r);
-    const dim3 grid((unsigned)std::min<int64_t>((f.dims[0] + 255) / 256, 1024), (unsigned)std::min<int64_t>(n, 32768));
-    if (TO_FIELD) PS_HIP(copy(g.p, host + (size_t)r * w, w * (size_t)n));
-#define PS_ROWS(T) hipLaunchKernelGGL((ps_rows_k<T, TO_FIELD>), grid, dim3(256), 0, st, (T*)f.ptr, (long long)f.dims[0], (long long)f.dims[1], (long long)f.pitch, (long long)f.plane, (long long)r, (long long)n, (T*)g.p)
-    if (es == 8) PS_ROWS(uint64_t);
-    else if (es == 4) PS_ROWS(uint32_t);
-    else if (es == 2) PS_ROWS(uint16_t);
-    else PS_ROWS(uint8_t);
-#undef PS_ROWS
-    PS_HIP(hipGetLastError());
-    if (!TO_FIELD) PS_HIP(copy(g.p, host + (size_t)r * w, w * (size_t)n));
-  }
-  PS_HIP(hipStreamSynchronize(st));
-  return 0;
-}
-
 extern "C" int ps_field_h2d(const ps_field* f, const void* host, void* stream) {
   if (int r = require_init()) return r;
-  return transfer<true>(data_of(*f), (char*)host, stream_of(stream));
+  return transfer(data_of(*f), (char*)host, stream_of(stream), true);
 }
 
 extern "C" int ps_field_d2h(const ps_field* f, void* host, void* stream) {
   if (int r = require_init()) return r;
-  return transfer<false>(data_of(*f), (char*)host, stream_of(stream));
+  return transfer(data_of(*f), (char*)host, stream_of(stream), false);
 }
 
 static unsigned grid_for(long long n) {

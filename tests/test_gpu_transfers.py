@@ -1,6 +1,6 @@
 """Host transfers of fields: dense rows (one copy), padded rows and views (through the dense block on the
 device), several pieces of the block, every element size, and several threads at once."""
-import threading
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -41,21 +41,17 @@ def test_views_touch_only_their_box(lo, hi):
 def test_threads_transfer_at_once():
     hs = [_host((100 + i, 50, 40), ps.Float64, i) for i in range(6)]
     fields = [ps.zeros(*h.shape, eltype=ps.Float64) for h in hs]
-    bad = []
 
     def work(i):
         st = ps.get_stream(1 + i % 3)
         for _ in range(4):
             fields[i].copy_from(hs[i], st)
             if not np.array_equal(fields[i].to_host(st), hs[i]):
-                bad.append(i)
+                return False
+        return True
 
-    ts = [threading.Thread(target=work, args=(i,)) for i in range(6)]
-    for t in ts:
-        t.start()
-    for t in ts:
-        t.join()
-    assert not bad
+    with ThreadPoolExecutor(6) as pool:  # result() raises what a worker raised
+        assert [f.result() for f in [pool.submit(work, i) for i in range(6)]] == [True] * 6
 
 
 @pytest.mark.parametrize("shape,et", [((1,), ps.Float64), ((1001,), ps.Float32), ((33, 3), ps.Float64), ((1025, 70, 1), ps.Float32), ((130, 9, 7), ps.BFloat16),
