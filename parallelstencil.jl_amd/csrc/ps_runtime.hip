@@ -679,8 +679,13 @@ struct Transfer {
     return nullptr;
   }
   static void free(char* p) { (void)hipFree(p); }
-  int copy(char* dev, char* h, size_t n) {
-    return done(to_field ? hipMemcpyAsync(dev, h, n, hipMemcpyHostToDevice, st) : hipMemcpyAsync(h, dev, n, hipMemcpyDeviceToHost, st));
+  // Up to 16 KiB to the host, or alone, as a strided copy of one row, which comes back sooner: 1 KiB to the
+  // host 10.6 us against 19.9 (to the device 10.8 and 13.0; in front of a kernel 24 and 18), 16 KiB 16.6 and
+  // 25.6, 64 KiB 37 and 34.
+  int copy(char* dev, char* h, size_t n, bool alone = false) {
+    const hipMemcpyKind kind = to_field ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
+    char *const d = to_field ? dev : h, *const s = to_field ? h : dev;
+    return done(n <= 16384 && (alone || !to_field) ? hipMemcpy2DAsync(d, n, s, n, n, 1, kind, st) : hipMemcpyAsync(d, s, n, kind, st));
   }
   int sync() { return done(hipStreamSynchronize(st)); }
   char* row(int64_t r) const { return (char*)f.ptr + ((r % f.dims[1]) * f.pitch + (r / f.dims[1]) * f.plane) * (int64_t)elsize(f.dtype); }
@@ -717,7 +722,7 @@ int transfer(const ps_field& f, char* host, hipStream_t st, bool to_field) {
   if (!f.ptr || !host) return fail(PS_EHIP, "invalid argument: a transfer needs device and host memory");
   Transfer t{f, st, to_field};
   if ((f.dims[1] == 1 || f.pitch == f.dims[0]) && (f.dims[2] == 1 || f.plane == f.dims[0] * f.dims[1])) {  // dense
-    const int rc = t.copy((char*)f.ptr, host, w * (size_t)rows);
+    const int rc = t.copy((char*)f.ptr, host, w * (size_t)rows, true);
     return rc ? rc : t.sync();
   }
   return transfer_rows(t, block_pool(), to_field, w, rows, host);
