@@ -269,6 +269,7 @@ struct Module {
   hipModule_t mod = nullptr;
   hipFunction_t fn = nullptr;
   Emitted em;
+  std::vector<char> code;  // the code object until it is loaded
 };
 
 struct LaunchEntry;
@@ -539,17 +540,25 @@ std::shared_ptr<Module> get_module(KernelObj* ko, const Kernel& K, const std::ve
   std::string key = kinds_key(kinds) + v.key();
   std::lock_guard<std::mutex> lk(ko->mu);
   auto it = ko->variants.find(key);
-  if (it != ko->variants.end() && (!load || it->second->fn)) return it->second;
-  auto m = std::make_shared<Module>();
-  m->em = lower_kernel(K, kinds, v);
-  std::vector<char> code = code_object(K, m->em);
-  if (load) {
-    hipError_t e = hipModuleLoadData(&m->mod, code.data());
+  std::shared_ptr<Module> m = it != ko->variants.end() ? it->second : nullptr;
+  if (!m) {
+    m = std::make_shared<Module>();
+    m->em = lower_kernel(K, kinds, v);
+    m->code = code_object(K, m->em);
+    ko->variants[key] = m;
+  }
+  if (load && !m->fn) {  // a variant compiled ahead is loaded as it is, not emitted again
+    hipError_t e = hipModuleLoadData(&m->mod, m->code.data());
     if (e != hipSuccess) throw PsError(PS_EHIP, std::string("hipModuleLoadData: ") + hipGetErrorString(e));
     e = hipModuleGetFunction(&m->fn, m->mod, m->em.entry.c_str());
+    if (e != hipSuccess) {
+      (void)hipModuleUnload(m->mod);
+      m->mod = nullptr;
+      m->fn = nullptr;
+    }
     if (e != hipSuccess) throw PsError(PS_EHIP, std::string("hipModuleGetFunction: ") + hipGetErrorString(e));
+    m->code = std::vector<char>();
   }
-  ko->variants[key] = m;
   return m;
 }
 
