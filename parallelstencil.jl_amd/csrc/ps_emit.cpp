@@ -2867,6 +2867,24 @@ int idx_span(const Kernel& K, int q) {
   return (int)span;
 }
 
+int value_quotients(const Kernel& K) {
+  std::function<bool(const NodeP&)> loads = [&](const NodeP& n) -> bool {
+    if (!n) return false;
+    if (n->k == NK::Index) return true;
+    for (auto& a : n->a)
+      if (loads(a)) return true;
+    return false;
+  };
+  int count = 0;
+  std::function<void(const NodeP&)> walk = [&](const NodeP& n) {
+    if (!n) return;
+    count += n->k == NK::Binary && n->s == "/" && loads(n->a[1]);
+    for (auto& a : n->a) walk(a);
+  };
+  walk(K.body);
+  return count;
+}
+
 bool only_writes(const Kernel& K) {
   std::function<bool(const NodeP&)> reads = [&](const NodeP& n) -> bool {
     if (!n) return false;

@@ -217,6 +217,9 @@ bool groupable_body(const Kernel& k, bool z = false);
 // array (0: no neighbours along q).
 int idx_span(const Kernel& k, int q);
 
+// Quotients in the body whose divisor reads an array element.
+int value_quotients(const Kernel& k);
+
 // Whether no statement of the body reads an array element (array assignments and their conditions).
 bool only_writes(const Kernel& k);
 std::string kernel_info_json(const Kernel& k);

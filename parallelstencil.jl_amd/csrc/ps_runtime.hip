@@ -1716,6 +1716,8 @@ Plan plan_launch(const Kernel& K, const ps_arg* args, int nargs, const ps_launch
       // 192^3 36.1 / 32.6, 255^3 107 / 87, 255x512x512 442 / 333; acoustic3D compute_V 160^3 46 / 41,
       // 192^3 86 / 67, 255x320x320 326 / 259, compute_P 0 to 10% faster). Shorter rows lose as often as
       // they gain: 100x255x255 compute_V 65 / 72, diffusion3D 49 / 37; 63x255x255 33 / 42 and 25 / 31.
+      // Not with several quotients by array values per cell, whose divisions bound the kernel (Stokes3D
+      // compute_timesteps, three: 160^3 36 / 47, 200x300x100 54 / 66, 191^3 66 / 74; diffusion3D has one).
       // 2 x cells pay from 12e6 cells on: 300x200x128 37.6 us with 1 x 4 and 40.6 with 2 x 4,
       // 512x100x40 12.1 and 12.7, 192x255x255 72.7 and 72.4, 255x512x512 349 and 333.
       const int64_t cells = len[0] * len[1] * len[2];
@@ -1723,7 +1725,7 @@ Plan plan_launch(const Kernel& K, const ps_arg* args, int nargs, const ps_launch
       // wave of one store is bound by the launch of waves (64^3 4.3 -> 3.7 us, 128^3 6.6 -> 5.6, 256^3
       // 30.3 -> 18.4, 512^3 224 -> 192; 2 z cells 3.8, 7.7, 28.1, 154 to 195; 2 x cells slower).
       const bool fill = es >= 8 && only_writes(K) && groupable_body(K, true);
-      const bool fp64 = es >= 8 && (len[0] >= 256 || (len[0] >= 160 && cells >= 4000000)) && groupable_body(K, true);
+      const bool fp64 = es >= 8 && (len[0] >= 256 || (len[0] >= 160 && cells >= 4000000 && value_quotients(K) <= 1)) && groupable_body(K, true);
       int cz = 1;
       if (K.opt.cells_z != 0) cz = K.opt.cells_z;
       else if (fill) cz = 4;

@@ -71,6 +71,21 @@ def test_kernels_without_reads_match_one_cell(src, shape):
         assert np.array_equal(x, y), shape
 
 
+@pytest.mark.parametrize("shape", [(160, 161, 157), (200, 170, 121), (257, 40, 33)])
+def test_quotients_by_values_match_one_cell(shape):
+    # several quotients by array values per cell: one cell per thread in rows below 256, z cells from there on
+    nx, ny, nz = shape
+    out = []
+    for kw in ({}, dict(cells_x=1, cells_z=1)):
+        k = ps.core._define("parallel", W.STOKES3D_TIMESTEPS, kw, M64)
+        D = [ps.zeros(*s) for s in ((nx - 1, ny - 2, nz - 2), (nx - 2, ny - 1, nz - 2), (nx - 2, ny - 2, nz - 1), shape)]
+        Mus = ps.zeros(*shape).copy_from(np.asfortranarray(1.0 + np.random.default_rng(nx).random(shape)))
+        k(*D, Mus, 1.0, 0.25, 1e-3, max(shape))
+        out.append([np.ascontiguousarray(d.to_host()).view(np.uint64) for d in D])
+    for x, y in zip(*out):
+        assert np.array_equal(x, y), shape
+
+
 def test_a_kernel_compiled_ahead_is_not_emitted_again():
     """The first launch after precompile_launch only loads the code object: emitting the grouped source again
     is more than half of what a first launch without it takes (880 us, 310 after precompile_launch)."""
