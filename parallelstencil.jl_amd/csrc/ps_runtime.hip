@@ -80,23 +80,23 @@ __global__ void __launch_bounds__(256) ps_fill_k(T* p, long long nx, long long n
   }
 }
 
-// Copies rows (row r: row r % ny of plane r / ny) of nv 16-byte pieces (0 where the rows are not so
-// aligned) and nt elements behind them. One element per thread with 64-bit index quotients took 5.5 us
-// for 1024^2 FP32, the rows by 16 bytes 3.4.
+// Copies nz x ny rows of nv 16-byte pieces (0 where the rows are not so aligned) and nt elements behind them:
+// blockIdx.x and threadIdx.x over the pieces, y over the rows, blockIdx.z over the planes. No index
+// quotients: a kernel this short is otherwise bound by fetching its own code (the 1 x 255 x 255 face of a
+// halo 3.6 us, 17 with the quotients of four rows unrolled).
 template <class T>
-__global__ void __launch_bounds__(256) ps_copy_k(T* __restrict__ d, const T* __restrict__ s, int64_t nv, int64_t nt, int64_t ny, int64_t rows,
+__global__ void __launch_bounds__(256) ps_copy_k(T* __restrict__ d, const T* __restrict__ s, int64_t nv, int64_t nt, int64_t ny, int64_t nz,
                                                  int64_t dsx, int64_t dsxy, int64_t ssx, int64_t ssxy) {
   constexpr int V = 16 / sizeof(T);
-  for (int64_t r = (int64_t)blockIdx.y * blockDim.y + threadIdx.y; r < rows; r += (int64_t)gridDim.y * blockDim.y) {
-    int64_t z = 0, y = r;
-    if (rows != ny) z = r / ny, y = r - z * ny;
-    T* const dr = d + y * dsx + z * dsxy;
-    const T* const sr = s + y * ssx + z * ssxy;
-    for (int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; x < nv + nt; x += (int64_t)gridDim.x * blockDim.x) {
-      if (x < nv) ((uint4*)dr)[x] = ((const uint4*)sr)[x];
-      else dr[nv * V + x - nv] = sr[nv * V + x - nv];
+  for (int64_t z = blockIdx.z; z < nz; z += gridDim.z)
+    for (int64_t y = (int64_t)blockIdx.y * blockDim.y + threadIdx.y; y < ny; y += (int64_t)gridDim.y * blockDim.y) {
+      T* const dr = d + y * dsx + z * dsxy;
+      const T* const sr = s + y * ssx + z * ssxy;
+      for (int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; x < nv + nt; x += (int64_t)gridDim.x * blockDim.x) {
+        if (x < nv) ((uint4*)dr)[x] = ((const uint4*)sr)[x];
+        else dr[nv * V + x - nv] = sr[nv * V + x - nv];
+      }
     }
-  }
 }
 
 __global__ void ps_set_i32_k(int* p, int v) { *p = v; }
@@ -921,13 +921,31 @@ extern "C" int ps_field_copy(const ps_field* dst_in, const ps_field* src_in, voi
   long long n = dst->dims[0] * dst->dims[1] * dst->dims[2];
   if (n == 0) return 0;
   const int64_t es = (int64_t)elsize(dst->dtype), rows = dst->dims[1] * dst->dims[2], w = dst->dims[0] * es;
-  // 16-byte pieces where every row of both starts on one
-  const bool v = (((uintptr_t)dst->ptr | (uintptr_t)src->ptr) & 15) == 0 &&
+  // 16-byte pieces where every row of both starts on one (short rows only if they end on one too)
+  const bool v = (w >= 128 || w % 16 == 0) && (((uintptr_t)dst->ptr | (uintptr_t)src->ptr) & 15) == 0 &&
                  (rows == 1 || ((dst->pitch | src->pitch | dst->plane | src->plane) * es) % 16 == 0);
   const int64_t nv = v ? w / 16 : 0, nt = (w - 16 * nv) / es;
-  const dim3 b = rows >= 4 ? dim3(64, 4) : dim3(256, 1);
-  const dim3 g((unsigned)std::min<int64_t>((nv + nt + b.x - 1) / b.x, 1 << 20), (unsigned)std::min<int64_t>((rows + b.y - 1) / b.y, 65535));
-#define PS_COPY(T) hipLaunchKernelGGL(ps_copy_k<T>, g, b, 0, st, (T*)dst->ptr, (const T*)src->ptr, nv, nt, (int64_t)dst->dims[1], rows, (int64_t)dst->pitch, (int64_t)dst->plane, (int64_t)src->pitch, (int64_t)src->plane)
+  // planes that follow each other at the pitch of the rows are rows of one plane; otherwise the longer of
+  // the two dimensions is the rows'
+  int64_t ny = dst->dims[1], nz = dst->dims[2], dsx = dst->pitch, dsxy = dst->plane, ssx = src->pitch, ssxy = src->plane;
+  if (dsxy == ny * dsx && ssxy == ny * ssx) ny *= nz, nz = 1;
+  if (ny < nz) std::swap(ny, nz), std::swap(dsx, dsxy), std::swap(ssx, ssxy);
+  // Threads along a row, a power of two; the block's others lie on further rows. 16-byte pieces: as many as
+  // the row has, up to 64 (256 for up to three rows). Single elements: up to 256, so that lines that two
+  // chunks of a row share stay in one block, and from 4096 blocks on four rows or planes per thread (510^3
+  // off a 16-byte boundary, FP64: 64 threads 500 us, 256 541, 256 and four rows 385; 65 025 rows of 33:
+  // 12.3 with one, 8.8 with four). 64 threads for any row took 38 us for the 1 x 512 x 512 face of a halo,
+  // as wide as the row 9.
+  const int64_t units = nv + nt, most = v && ny >= 4 ? 64 : 256;
+  unsigned bx = 1;
+  while (bx < most && bx < units) bx *= 2;
+  const dim3 b(bx, 256 / bx);
+  // a last chunk of less than a quarter of the threads is the first block's second turn
+  const int64_t gx = std::min<int64_t>(std::max<int64_t>(units / bx + (units % bx > bx / 4), 1), 1 << 20);
+  int64_t gy = (ny + b.y - 1) / b.y, gz = nz;
+  if (!v && gx * gy * gz >= 4096) (gy >= 16 ? gy : gz) = ((gy >= 16 ? gy : gz) + 3) / 4;
+  const dim3 g((unsigned)gx, (unsigned)std::min<int64_t>(gy, 65535), (unsigned)std::min<int64_t>(gz, 65535));
+#define PS_COPY(T) hipLaunchKernelGGL(ps_copy_k<T>, g, b, 0, st, (T*)dst->ptr, (const T*)src->ptr, nv, nt, ny, nz, dsx, dsxy, ssx, ssxy)
   if (es == 8) PS_COPY(long long);
   else if (es == 4) PS_COPY(int);
   else if (es == 2) PS_COPY(unsigned short);

@@ -55,7 +55,8 @@ def test_threads_transfer_at_once():
 
 
 @pytest.mark.parametrize("shape,et", [((1,), ps.Float64), ((1001,), ps.Float32), ((33, 3), ps.Float64), ((1025, 70, 1), ps.Float32), ((130, 9, 7), ps.BFloat16),
-                                      ((65, 1, 9), ps.Bool), ((2, 70000), ps.Float64)])
+                                      ((65, 1, 9), ps.Bool), ((2, 70000), ps.Float64), ((1, 9, 7001), ps.Float32), ((7, 3, 9000), ps.Float64),
+                                      ((17, 5, 4099), ps.BFloat16), ((5, 3), ps.Bool), ((1030, 2), ps.Float64), ((3, 70000, 2), ps.Int32)])
 def test_device_copies(shape, et):
     h = _host(shape, et, 4)
     A, B = ps.zeros(*shape, eltype=et).copy_from(h), ps.zeros(*shape, eltype=et)
@@ -63,7 +64,8 @@ def test_device_copies(shape, et):
     assert np.array_equal(B.to_host(), h)
 
 
-@pytest.mark.parametrize("lo,hi", [((2, 1, 1), (33, 20, 9)), ((5, 3, 2), (30, 19, 8)), ((3, 4, 5), (3, 20, 5))])
+@pytest.mark.parametrize("lo,hi", [((2, 1, 1), (33, 20, 9)), ((5, 3, 2), (30, 19, 8)), ((3, 4, 5), (3, 20, 5)), ((1, 1, 1), (1, 20, 9)),
+                                   ((32, 1, 1), (33, 20, 9)), ((2, 5, 2), (9, 5, 8)), ((4, 2, 3), (4, 2, 3))])
 def test_device_copies_of_views(lo, hi):
     # rows that start off a 16-byte boundary, and elements beside the view that must stay
     ha, hb = _host((33, 20, 9), ps.Float64, 5), _host((40, 21, 9), ps.Float64, 6)
