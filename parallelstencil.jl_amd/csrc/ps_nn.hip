@@ -876,7 +876,8 @@ int gemm_launch(int M, int N, int K, const void* A, int64_t sam, int64_t sak, co
   if (M == 0 || N == 0) return 0;
   if ((epi == PS_NN_EPI_BF16_BIAS_RELU || epi == PS_NN_EPI_BF16_BIAS) && !bias) return ps_internal_fail(PS_EARGUMENT, "ps_nn_gemm: bias missing");
   if (splitk > 1 && epi != PS_NN_EPI_F32_ADD) return ps_internal_fail(PS_EARGUMENT, "ps_nn_gemm: split-K needs the accumulating FP32 epilogue");
-  if (AM == 0 && splitk == 1 && N <= THIN && K <= THIN_K && K % 8 == 0 && K > 0 && sak == 1 && sam % 8 == 0 && ((uintptr_t)A & 15) == 0 && epi <= PS_NN_EPI_BF16_BIAS &&
+  // K of a multiple of 72 may be the columns of a 3x3 im2col, whose product is that of the convolution bit for bit
+  if (AM == 0 && splitk == 1 && N <= THIN && K <= THIN_K && K % 8 == 0 && K % 72 != 0 && K > 0 && sak == 1 && sam % 8 == 0 && ((uintptr_t)A & 15) == 0 && epi <= PS_NN_EPI_BF16_BIAS &&
       epi >= 0) {
     const dim3 g((unsigned)((M + 255LL) / 256));
 #define NN_THIN(E) hipLaunchKernelGGL((nn_thin_n_k<E>), g, dim3(256), 0, st, (long long)M, N, K, (const bf16_t*)A, sam, (const bf16_t*)B, sbk, sbn, (bf16_t*)C, ldc, bias)
