@@ -892,9 +892,14 @@ int gemm_launch(int M, int N, int K, const void* A, int64_t sam, int64_t sak, co
                        sbn, (bf16_t*)C, ldc);
     return launched("ps_nn_gemm");
   }
-  if (AM == 0 && splitk > 1 && N <= THIN && M % 8 == 0 && M <= 2048 && sam == 1 && sak % 8 == 0 && ((uintptr_t)A & 15) == 0 && sbn == 1 && K > 0) {
-    // the epilogue is the accumulating one here; about one workgroup per CU, 256 rows at least
-    const long long chunk = std::max<long long>(256, (K + 255LL) / 256);
+  // Not where the split already leaves the MFMA product short sums (64 rows of 600 pixels, split 64: 5.3 us
+  // there, 6.3 here, split 2 12.3; 1024 of 16384, split 64: 22 and 28, split 8 69, split 512 55), nor for
+  // many rows of few pixels (2048 of 4096: 14 to 66 us there, 116 here).
+  if (AM == 0 && splitk > 1 && N <= THIN && M % 8 == 0 && sam == 1 && sak % 8 == 0 && ((uintptr_t)A & 15) == 0 && sbn == 1 &&
+      (M <= 256 ? K > 2048 || K > 128LL * splitk : M <= 2048 && K >= 16384 && (K < 64LL * splitk || K > 1024LL * splitk))) {
+    // the epilogue is the accumulating one here; about one workgroup per CU, each with 256 rows, or where
+    // the pieces of a row leave fewer than 64 of them to be summed at a time, four per thread
+    const long long chunk = std::max<long long>(std::min(256, 4 * (256 / (M / 8))), (K + 255LL) / 256);
     hipLaunchKernelGGL(nn_thin_grad_k, dim3((unsigned)((K + chunk - 1) / chunk)), dim3(256), 0, st, M, N, (long long)K, (const bf16_t*)A, sak, (const bf16_t*)B, sbk,
                        (float*)C, ldc, chunk);
     return launched("ps_nn_gemm");

@@ -178,7 +178,8 @@ def test_thin_sums_against_float64(M, N, K):
     assert (np.abs(C.download() - ref) <= 2.0 ** -8 * np.abs(ref) + 2.0 ** -20).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(8, 1, 300), (32, 3, 131072), (24, 4, 1000), (2048, 2, 700), (2056, 2, 700)])
+@pytest.mark.parametrize("M,N,K", [(8, 1, 300), (32, 3, 131072), (24, 4, 1000), (2048, 2, 700), (2056, 2, 700), (64, 3, 50), (256, 3, 600), (256, 4, 70000),
+                                   (264, 1, 4000), (8, 4, 5)])
 def test_thin_gradients_against_float64(M, N, K):
     rng = np.random.default_rng(M + N + K)
     a, d = _bf(rng.standard_normal((K, M))), _bf(rng.standard_normal((K, N)))
