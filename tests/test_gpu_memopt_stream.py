@@ -1,7 +1,8 @@
-"""memopt streams against plain kernels, bit for bit, over the grids where the number of planes per
-thread changes (2, 4, 8, 16 and 32, and remainders of each), for a stencil and for in-place updates read
-ahead; quotients of one scalar by an array taken once per value; the gather form of a derivative with
-its streams against the atomic scatter form."""
+"""memopt streams against plain kernels, bit for bit, over the grids where the automatic number of planes per
+thread changes (2, 4 and 8, with remainders), with 16 and 32 planes given (which the automatic choice takes
+from 33 and 67 million cells on), in two and three dimensions and every floating-point type: a stencil,
+in-place updates read ahead, quotients of one scalar by an array taken once per value, and the gather form of
+a derivative; the latter against the atomic scatter form too."""
 import numpy as np
 import pytest
 
@@ -94,6 +95,87 @@ def test_gather_matches_scatter(dims, memopt):
     # seven products a cell, each a few roundings, in either order: 1e-14 of the largest term (about 5)
     assert np.abs(outs[0][1] - outs[1][1]).max() <= 1e-13
 
+
+NP = {ps.Float64: np.float64, ps.Float32: np.float32, ps.BFloat16: np.float32}
+STENCIL2D = """
+@parallel function stencil2d!(T2, T, Ci, lam, dt, dx, dy)
+    @inn(T2) = @inn(T) + dt*(lam*@inn(Ci)*(@d2_xi(T)/dx/dx + @d2_yi(T)/dy/dy))
+    return
+end
+"""
+QUOT2D = """
+@parallel_indices (ix,iy) function quotients2d!(B, A, C, s)
+    if (1 < ix < size(A,1) && 1 < iy < size(A,2))
+        B[ix,iy] = B[ix,iy] + A[ix-1,iy]*(s/C[ix-1,iy]) + A[ix+1,iy]*(s/C[ix+1,iy]) - A[ix,iy-1]*(s/C[ix,iy-1]) + s/C[ix,iy+1]
+    end
+    return
+end
+"""
+ACOUSTIC2D = """
+@parallel function step2d!(P, Vx, Vy, dt, k, dx, dy)
+    @all(P) = @all(P) - dt*k*(@d_xa(Vx)/dx + @d_ya(Vy)/dy)
+    return
+end
+"""
+
+
+def _field(dims, et, seed, lo=0.0):
+    h = (lo + np.random.default_rng(seed).random(dims)).astype(np.float32 if et != ps.Float64 else np.float64)
+    return ps.zeros(*dims, eltype=et).copy_from(ps.f32_to_bf16(h) if et == ps.BFloat16 else h)
+
+
+def _module(et, nd):
+    mod = f"{MOD}.{et}.{nd}"
+    if not ps.is_initialized(mod):
+        ps.init_parallel_stencil(ps.AMDGPU, ps.Float64 if et == ps.Float64 else ps.Float32, nd, module=mod)
+    return mod
+
+
+@pytest.mark.parametrize("loopsize", [None, 16, 32])
+@pytest.mark.parametrize("et", [ps.Float64, ps.Float32, ps.BFloat16])
+@pytest.mark.parametrize("dims", [(20, 17), (256, 130), (257, 131), (96, 515), (1030, 1021), (64, 20, 70), (33, 19, 40), (130, 61, 45)])
+def test_types_and_dimensions_match_plain(dims, et, loopsize):
+    nd, t = len(dims), NP[et]
+    mod = _module(et, nd)
+    kw = {} if loopsize is None else {"loopsize": loopsize}
+    stag = [tuple(n + (i == d) for i, n in enumerate(dims)) for d in range(nd)]
+    outs = []
+    for memopt in (False, True):
+        opts = dict(kw, memopt=True) if memopt else {}
+        d = lambda kind, text: ps.core._define(kind, text, opts, mod)  # noqa: B023, E731
+        kst = d("parallel", STENCIL2D) if nd == 2 else d("parallel", W.DIFFUSION3D)
+        kq = d("parallel_indices", QUOT2D if nd == 2 else QUOT)
+        kp = d("parallel", ACOUSTIC2D) if nd == 2 else d("parallel", W.ACOUSTIC3D_P)
+        steps = [t(v) for v in (0.1, 0.2, 0.3)[:nd]]
+        T2, B, P, S, R = (_field(dims, et, i) for i in range(5))
+        T, C = _field(dims, et, 5), _field(dims, et, 6, 0.5)
+        kst(T2, T, C, t(1.1), t(0.001), *steps)
+        if dims in ((20, 17), (256, 130), (96, 515), (64, 20, 70)):  # sizes that a block divides: a memopt kernel with indices refuses others
+            kq(B, T, C, t(0.7))
+        for _ in range(2):
+            kp(P, *(_field(s, et, 7 + i) for i, s in enumerate(stag)), t(0.01), t(0.9), *steps)
+        g = kst._derivative("Reverse", {"T2": "DuplicatedNoNeed", "T": "DuplicatedNoNeed"})._gather[0]
+        assert g.info["memopt"] is memopt
+        ps.core.Kernel.__call__(g, T2, T, C, t(1.1), t(0.001), *steps, S, R)
+        outs.append([A.to_host() for A in (T2, B, P, R)])
+    for name, a, b in zip(("stencil", "quotients", "in place", "gather"), *outs):
+        assert np.array_equal(a, b), name
+
+
+@pytest.mark.parametrize("loopsize", [16, 32])
+@pytest.mark.parametrize("dims", [(20, 17, 9), (64, 64, 33), (127, 95, 63), (200, 130, 61)])
+def test_gather_with_long_streams_matches_scatter(dims, loopsize):
+    k = W.define_diffusion3d(True, MOD, loopsize=loopsize)
+    d = k._derivative("Reverse", {"T2": "DuplicatedNoNeed", "T": "DuplicatedNoNeed"})
+    T, T2, Cp = _rand(dims, 1), _rand(dims, 2), _rand(dims, 3, 1.0)
+    outs = []
+    for gather in (False, True):
+        S, R = _rand(dims, 4, -0.5), _rand(dims, 5)
+        d.use_gather = gather
+        d(T2, T, Cp, 1.1, 0.01, 0.1, 0.2, 0.3, S, R)
+        outs.append((S.to_host(), R.to_host()))
+    assert np.array_equal(outs[0][0], outs[1][0])
+    assert np.abs(outs[0][1] - outs[1][1]).max() <= 1e-13  # as in test_gather_matches_scatter
 
 INDIRECT = """
 @parallel_indices (ix,iy,iz) function indirect!(B, C, I, s)

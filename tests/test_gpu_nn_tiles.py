@@ -19,17 +19,46 @@ def _bf(a):
 
 
 # image sizes around the 8- and 16-column tiles, channels around the groups of 8 and 32 and beyond what
-# fits two patches (and one patch) into LDS, output channels around 32 and 64
+# one patch in LDS holds, output channels around 32 and 64. These take the tile of 128 x 32 (or the general
+# product), as their tiles are fewer than the CUs, but for 1 x 300 x 260, 32 -> 32.
 CONV = [(1, 1, 1, 8, 8), (2, 15, 17, 32, 33), (1, 16, 16, 24, 31), (3, 9, 8, 40, 65), (1, 33, 31, 7, 4), (2, 20, 24, 128, 130), (1, 70, 70, 96, 32),
         (4, 64, 64, 192, 64), (1, 10, 40, 384, 96), (1, 12, 12, 512, 16), (1, 300, 260, 32, 32), (2, 5, 100, 9, 12), (1, 17, 130, 2, 3), (2, 21, 37, 3, 40)]
-
-
+# the other tiles, which need that many pixels: 256 x 64, 128 x 64 and 256 x 32, each with whole and ragged
+# sizes and with channels that are multiples of 32, multiples of 8 and (256 x 32) neither
+LARGE = [(1, 256, 256, 192, 64), (3, 130, 170, 160, 70), (2, 200, 180, 136, 70), (8, 64, 64, 192, 64), (1, 128, 128, 384, 128), (2, 150, 130, 168, 40),
+         (1, 150, 150, 264, 130), (2, 181, 190, 64, 33), (2, 180, 200, 24, 20), (1, 260, 300, 3, 20)]
 # few output channels: the explicit product of so thin a side must not take another order of summation (BF16
 # results show one in about ten thousand sums)
 THIN_OUT = [(1, 300, 301, 8, 1), (2, 130, 130, 24, 3), (1, 201, 190, 32, 3), (1, 160, 170, 56, 4), (1, 16, 16, 40, 2)]
 
 
-@pytest.mark.parametrize("B,H,W,C,N", CONV + THIN_OUT)
+def _tile(B, H, W, C, N):
+    """(pixels, channels) of the convolution's tile, None for the general product, and the kind of its
+    channels: the rule of conv3_launch restated."""
+    up = lambda a, b: -(-a // b)  # noqa: E731
+
+    def fits(pix, nb):
+        w16, w8 = up(W, 16) * up(H, pix // 16), up(W, 8) * up(H, pix // 8)
+        lg = 3 if w8 < w16 else 4
+        stride = (C // 8 | 1) * 8 if C % 8 == 0 else C
+        return min(w16, w8) * B, 2 * (2 * 64 * (nb + 8) + ((pix >> lg) + 2) * ((1 << lg) + 2) * stride)
+
+    tiles = [(256, 64), (128, 64), (256, 32), (128, 32)]
+    for t in tiles[2 if fits(256, 32)[1] <= 80 << 10 else 0:]:
+        n, lds = fits(*t)
+        if lds <= 160 << 10 and (t == (128, 32) or n * up(N, t[1]) >= 256):
+            return t, "odd" if C % 8 else "32" if C % 32 == 0 else "8"
+    return None, None
+
+
+def test_the_lists_reach_every_tile():
+    taken = {_tile(*c) for c in CONV + LARGE}
+    assert taken >= {((256, 64), "32"), ((256, 64), "8"), ((128, 64), "32"), ((128, 64), "8"), ((256, 32), "32"), ((256, 32), "8"), ((256, 32), "odd"),
+                     ((128, 32), "32"), ((128, 32), "8"), ((128, 32), "odd"), (None, None)}
+    assert all(_tile(*c)[0] not in ((128, 32), None) for c in LARGE)
+
+
+@pytest.mark.parametrize("B,H,W,C,N", CONV + LARGE + THIN_OUT)
 def test_convolution_matches_the_column_matrix(B, H, W, C, N):
     rng = np.random.default_rng(B * H * W + C + N)
     P, K = B * H * W, 9 * C
@@ -85,8 +114,10 @@ def test_convolution_of_infinities_and_nan(special):
 
 @pytest.mark.parametrize("B,H,W,C,N", CONV)
 def test_weight_gradient_against_float64(B, H, W, C, N):
-    """FP32 sums of P products of BF16 values in any order: within P eps of the sum of magnitudes in
-    the worst case; sqrt(P) growth with a factor 8 is far inside it and far above what is seen."""
+    """FP32 sums of P products of BF16 values in any order are within P eps of the sum of magnitudes in the
+    worst case, about 0.64 P here; the bound of 8 eps (P + 4 sqrt P), linear in P, is that of eight roundings
+    of the sum of magnitudes (pixels of a tile, tiles of a workgroup, wavefronts, workgroups), as the sums
+    are taken in pieces."""
     rng = np.random.default_rng(B + H + W + C + N)
     P, K = B * H * W, 9 * C
     xh, dh = _bf(rng.standard_normal((B, H, W, C))), _bf(rng.standard_normal((P, N)))

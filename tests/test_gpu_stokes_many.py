@@ -29,8 +29,8 @@ def _start(sv, seed, scale=1.0):
     sv.reset(*(scale * (rng.random(A.shape) - 0.5) for A in (sv.Vx, sv.Vy, sv.Pt)))
 
 
-# tiles of 8 up to 127 x 127 (16 x 16 = 256 of them), of 16 from 128 x 127 on, of 24 from 199 x 257, of 32 from 384 x 383
-@pytest.mark.parametrize("nx,ny,n", [(8, 8, 2), (9, 31, 3), (33, 8, 16), (127, 127, 17), (128, 127, 33), (199, 257, 9), (255, 260, 8),
+# tiles of 8 up to 127 x 127 (16 x 16 = 256 of them), of 16 from 128 x 127 to 255 x 255, of 24 to 383 x 383, of 32 beyond
+@pytest.mark.parametrize("nx,ny,n", [(8, 8, 2), (9, 31, 3), (33, 8, 16), (127, 127, 17), (128, 127, 33), (199, 257, 9), (255, 260, 8), (300, 310, 6), (383, 383, 9),
                                      (383, 100, 7), (384, 383, 5), (511, 390, 11), (70, 1100, 4)])
 def test_many_iterations_match_single_ones(nx, ny, n):
     a, b = (F.Stokes2DFused(MOD, nx, ny, graph=False, eta_ts="maxV") for _ in range(2))
