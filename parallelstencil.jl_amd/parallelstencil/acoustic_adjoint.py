@@ -153,7 +153,8 @@ class Acoustic2DInversion:
         self.snap = [(z(nx + 1, ny), z(nx, ny + 1)) for _ in range(self.seg)]
         # numbertype scalars
         self._t = np.float32 if core._numbertype_of(module) == core.Float32 else np.float64
-        self._plans = {}  # group -> (what its launches are bound to, {(step, default stream): prepared launch})
+        self._plans = {}  # prepared launches by (group, step, default stream)
+        self._bound = {}  # group -> what its launches are bound to
 
     def _follow(self):
         """Drops the prepared launches bound to anything that has changed since they were made: the scalars
@@ -173,19 +174,19 @@ class Acoustic2DInversion:
             "lV": (self.k_av, adj, self.K, bits(s.dt, s.dx, s.dy)),
             "lP": (self.k_ap, adj, bits(s.dt, s.rho, s.dx, s.dy)),
         }
-        for group, bound in now.items():
-            if group not in self._plans or self._plans[group][0] != bound:
-                self._plans[group] = (bound, {})
+        changed = {g for g, bound in now.items() if self._bound.get(g) != bound}
+        if changed:
+            self._plans = {k: L for k, L in self._plans.items() if k[0] not in changed}
+            self._bound = now
 
     def _run(self, group, n, make):
         """Runs the prepared launch of step n (None: the same for all steps) of `group` on the current
         default stream, made by make() on first use: a step of this model takes a few microseconds, less than
         building its argument blocks anew."""
-        plans = self._plans[group][1]
-        key = (n, core._stream_handle(None))
-        L = plans.get(key)
+        key = (group, n, core._stream_handle(None))
+        L = self._plans.get(key)
         if L is None:
-            L = plans[key] = make()
+            L = self._plans[key] = make()
         L()
 
     # -------------------------------------------------------------- forward
