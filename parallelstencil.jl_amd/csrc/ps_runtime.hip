@@ -1588,6 +1588,9 @@ Plan plan_launch(const Kernel& K, const ps_arg* args, int nargs, const ps_launch
   // us with 2 / 4 / 8 / 16 / 32 planes, diffusion3D FP64: 32^3 4.0 / 4.9 / 7.6 / 13.5 / 21.3, 64^3 3.9 / 5.1 / 7.7 / 12.8 /
   // 23.3, 128^3 14.2 / 13.0 / 13.7 / 16.9 / 27.5, 512 x 100 x 40 15.1 / 12.9 / 13.2 / 20.6 / 37.3, 256^3 95 / 84.5 / 83.0 /
   // 83.5 / 88.8 (its reverse mode 141 / 126 / 123 / 120 / 142), 512^3 768 / 666 / 612 / 614 / 602.
+  // 2-D and the narrower types alike: 5-point diffusion 512^2 4.5 / 4.9 / 5.8 / 8.0 / 12.9, 1024^2 7.5 / 7.0 / 7.3 / 9.9 /
+  // 14.2, 4096^2 98 / 88 / 88 / 97 / 96, FP32 43 / 40 / 40 / 42 / 43.5; acoustic3D compute_V 256^3 FP32 119 / 110 /
+  // 112 / 118 / 126, BF16 105 / 84 / 77 / 79 / 85.
   int stream = 0;
   if (memopt && !user_geom && !K.opt.loopsize_given && P.nthreads[K.mm.loopdim - 1] == 1) {
     const int Ld = K.mm.loopdim - 1;
