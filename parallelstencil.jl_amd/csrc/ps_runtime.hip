@@ -342,17 +342,16 @@ const std::string& cache_dir() {
   return s.cache_dir;
 }
 
-unsigned long long fnv1a(const std::string& x, unsigned long long h = 1469598103934665603ULL) {
-  for (unsigned char c : x) {
-    h ^= c;
-    h *= 1099511628211ULL;
-  }
-  return h;
-}
-
+// Two 64-bit FNV-1a hashes from different starts, side by side: each step waits for a multiplication, and the
+// source of a kernel in groups of cells has 50 000 to 80 000 of them.
 std::string hash_hex(const std::string& x) {
+  unsigned long long h = 1469598103934665603ULL, g = 0x84222325cbf29ce4ULL;
+  for (unsigned char c : x) {
+    h = (h ^ c) * 1099511628211ULL;
+    g = (g ^ c) * 1099511628211ULL;
+  }
   char b[40];
-  std::snprintf(b, sizeof b, "%016llx%016llx", fnv1a(x), fnv1a(x, 0x84222325cbf29ce4ULL));
+  std::snprintf(b, sizeof b, "%016llx%016llx", h, g);
   return b;
 }
 
@@ -384,10 +383,11 @@ std::vector<char> code_object(const Kernel& K, const Emitted& em) {
   key += "\n//hiprtc " + std::to_string(vmaj) + "." + std::to_string(vmin);
   std::string path = cache_dir() + "/" + hash_hex(key) + ".hsaco";
   {
-    std::ifstream f(path, std::ios::binary);
-    if (f) {
-      std::vector<char> buf((std::istreambuf_iterator<char>(f)), std::istreambuf_iterator<char>());
-      if (!buf.empty()) return buf;
+    std::ifstream f(path, std::ios::binary | std::ios::ate);
+    const std::streamoff size = f ? (std::streamoff)f.tellg() : 0;
+    if (size > 0) {
+      std::vector<char> buf((size_t)size);
+      if (f.seekg(0).read(buf.data(), size)) return buf;
     }
   }
   hiprtcProgram prog;
