@@ -88,7 +88,7 @@ def test_quotients_by_values_match_one_cell(shape):
 
 def test_a_kernel_compiled_ahead_is_not_emitted_again():
     """The first launch after precompile_launch only loads the code object: emitting the grouped source again
-    is more than half of what a first launch without it takes (880 us, 310 after precompile_launch)."""
+    is more than half of what a first launch without it takes (810 us, 310 after precompile_launch)."""
     A = [ps.zeros(253, 190, 127) for _ in range(3)]
     args = (*A, 1.0, 0.1, 0.1, 0.1, 0.1)
 
